@@ -187,6 +187,200 @@ __global__ __launch_bounds__(64) void lm_head_ring(float *logits, unsigned long 
     if (best) publish_argmax(valid ? argmax_key(acc, n) : 0ull, best, m, slots);
 }
 
+// Several rows of x at once: the products on the matrix cores, the adds on the
+// vector ALUs. The reference's order is a product rounded, then an add rounded,
+// k in order: no fused multiply-add can give it, but a matrix instruction of
+// one k with a zero accumulator is the rounded product (a * b + 0; a product of
+// -0 becomes +0, and no partial sum is ever -0, so adding either leaves the
+// same bits), for 64 table rows and T rows of x at once. What is left for the
+// vector ALU is the one add a product needs, which bounds it: 128 rows of the
+// model's head are 17.4 G adds, 443 us at 64 lanes a cycle a CU; measured 579 us,
+// where a launch of one-row waves, each reading the table anew, took 10,160.
+// (32 rows a wave, a 32 x 32 instruction: 611; without the products issued a step
+// ahead: 592, and 355 against 248 us where a wave runs alone on its SIMD.)
+//
+// One wave owns a 64-row block of the table and MG times T rows of x. The packed
+// layout is the instruction's first operand as it stands (lane l: row l, four
+// consecutive k a 16-byte load), so table values go from memory to registers,
+// kRing 1-KB loads ahead; x goes through LDS, 64 k a stage, shared by the
+// workgroup's four waves. A lane ends with quads of 4 consecutive table rows of
+// one row of x: 16-byte stores.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// The products of one k: `of` gives the lane kQuads quads, quad q holding
+// table rows row(q, lane) .. + 3 of the block for row x_row(lane) of x.
+template <int T>
+struct Products;
+
+template <>
+struct Products<16> {
+    typedef f32x16 type;
+    static constexpr int kQuads = 4, kAhead = 1, kRing = 8;
+    static __device__ __forceinline__ type of(float w, float x) {
+        return __builtin_amdgcn_mfma_f32_16x16x1f32(w, x, type{}, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int q, int lane) { return 16 * q + 4 * (lane >> 4); }
+};
+
+template <>
+struct Products<4> {
+    typedef f32x4 type;
+    static constexpr int kQuads = 1, kAhead = 3, kRing = 16;
+    static __device__ __forceinline__ type of(float w, float x) {
+        return __builtin_amdgcn_mfma_f32_4x4x1f32(w, x, type{}, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int, int lane) { return 4 * (lane >> 2); }
+};
+
+template <int T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void head_rows(
+    float *logits, unsigned long long *__restrict__ best, const float *__restrict__ x,
+    const float4 *__restrict__ packed, int M, int64_t V, int H, const float *__restrict__ bias, const float *residual,
+    int slots) {
+    typedef Products<T> P;
+    constexpr int K4S = 16;                           // 16-byte pieces of k a stage
+    constexpr int STRIDE = 4 * K4S + 4;               // an x row in LDS: T rows' pieces on distinct banks
+    constexpr int PIECES = T * K4S, PER = (PIECES + 255) / 256;
+    constexpr int kRing = P::kRing, kAhead = P::kAhead;
+    static_assert(K4S % kRing == 0, "ring slots fixed per unrolled step");
+    __shared__ __align__(16) float sx[2][T * STRIDE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // workgroup i runs on XCD i mod 8: each XCD takes a contiguous range of tiles, the row tiles
+    // of one table range together, so the table is read from memory once for all of them
+    const int mtiles = (M + T - 1) / T, total = gridDim.x, full = total & ~7, id = blockIdx.x;
+    const int t = id < full ? (id & 7) * (total >> 3) + (id >> 3) : id;
+    const int m0 = (t % mtiles) * T;
+    const int64_t blk = (int64_t)(t / mtiles) * 4 + wave, blocks = (V + 63) / 64;
+    const int K4 = H / 4;
+    // the block's piece k4 as a buffer load: the piece is a scalar offset (no vector address
+    // arithmetic beside the adds), and one past the block's end reads as zero
+    const auto e = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float4 *>(packed) + min(blk, blocks - 1) * K4 * 64, 0, K4 * 1024, 0x00020000);
+    auto piece = [&](int at) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(e, lane * 16, at * 1024, 0));
+    };
+    f32x4 ring[kRing];
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) ring[i] = piece(i);
+
+    f32x4 held[PER];
+    auto fetch = [&](int k4) {                        // rows and pieces clamped in bounds; those past the
+#pragma unroll                                        // edges are never multiplied or never stored
+        for (int i = 0; i < PER; ++i) {
+            const int u = min((int)threadIdx.x + 256 * i, PIECES - 1);
+            held[i] = *reinterpret_cast<const f32x4 *>(x + (size_t)min(m0 + u / K4S, M - 1) * H +
+                                                       4 * min(k4 + u % K4S, K4 - 1));
+        }
+    };
+    auto keep = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int u = min((int)threadIdx.x + 256 * i, PIECES - 1);
+            *reinterpret_cast<f32x4 *>(&sx[buf][(u / K4S) * STRIDE + 4 * (u % K4S)]) = held[i];
+        }
+    };
+    typename P::type acc = {};
+    const float *xrow = &sx[0][(lane & (T - 1)) * STRIDE];
+
+    fetch(0);
+    keep(0);
+    __syncthreads();
+    int k4 = 0, buf = 0;
+    for (; k4 + K4S <= K4; k4 += K4S, buf ^= 1) {
+        fetch(k4 + K4S);
+        // The products of step j + kAhead are issued before the adds of step j (the scheduler, left to
+        // itself, waits for each product where it is issued), so a wave alone on its SIMD keeps both
+        // units busy; x is read from LDS a piece ahead.
+        const float *xs = xrow + buf * T * STRIDE;
+        f32x4 w = {}, xv = {}, xnext = *reinterpret_cast<const f32x4 *>(xs);
+        typename P::type prod[kAhead + 1];
+#pragma unroll
+        for (int j = 0; j < 4 * K4S + kAhead; ++j) {
+            if (j < 4 * K4S) {
+                if (j % 4 == 0) {
+                    w = ring[(j / 4) % kRing];
+                    ring[(j / 4) % kRing] = piece(k4 + j / 4 + kRing);
+                    xv = xnext;
+                    if (j + 4 < 4 * K4S) xnext = *reinterpret_cast<const f32x4 *>(xs + j + 4);
+                }
+                prod[j % (kAhead + 1)] = P::of(w[j % 4], xv[j % 4]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (j >= kAhead) acc += prod[(j - kAhead) % (kAhead + 1)];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        keep(buf ^ 1);
+        __syncthreads();
+    }
+    for (int i = 0; k4 + i < K4; ++i) {               // H not a multiple of 64
+        const f32x4 w = piece(k4 + i);
+        const f32x4 xv = *reinterpret_cast<const f32x4 *>(xrow + buf * T * STRIDE + 4 * i);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc += P::of(w[c], xv[c]);
+    }
+
+    if (blk >= blocks) return;
+    const bool vec = (V & 3) == 0 && ((uintptr_t)logits & 15) == 0 && ((uintptr_t)residual & 15) == 0;
+    const int m = m0 + (lane & (T - 1));
+    unsigned long long key = 0ull;
+#pragma unroll
+    for (int q = 0; q < P::kQuads; ++q) {
+        const int64_t n = blk * 64 + P::row(q, lane);
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[r] = acc[4 * q + r];
+            if (best && n + r < V) {
+                const unsigned long long mine = argmax_key(v[r], n + r);
+                key = mine > key ? mine : key;
+            }
+        }
+        if (!logits || m >= M) continue;
+        float *out = logits + (size_t)m * V + n;
+        if (vec && n < V) {
+            if (bias)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = __fadd_rn(v[r], bias[n + r]);
+            if (residual) {
+                const float4 res = *reinterpret_cast<const float4 *>(residual + (size_t)m * V + n);
+                v[0] = __fadd_rn(res.x, v[0]);
+                v[1] = __fadd_rn(res.y, v[1]);
+                v[2] = __fadd_rn(res.z, v[2]);
+                v[3] = __fadd_rn(res.w, v[3]);
+            }
+            *reinterpret_cast<float4 *>(out) = make_float4(v[0], v[1], v[2], v[3]);
+        } else if (!vec) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < V) out[r] = head_epilogue(v[r], m, n + r, V, bias, residual);
+        }
+    }
+    if (best) {                                       // the lanes holding one row of x: T apart
+#pragma unroll
+        for (int off = 32; off >= T; off >>= 1) {
+            const unsigned long long other = __shfl_xor(key, off, 64);
+            key = other > key ? other : key;
+        }
+        if (lane < T && m < M) {
+            if (slots)
+                best[(int64_t)m * slots + blk] = key;
+            else if (key != 0ull)
+                atomicMax(best + m, key);
+        }
+    }
+}
+
+template <int T>
+int32_t launch_head_rows(void **p, const int64_t *s, int slots) {
+    const int64_t tiles = ((s[0] + T - 1) / T) * (((s[1] + 63) / 64 + 3) / 4);
+    hipLaunchKernelGGL((head_rows<T>), dim3((unsigned)tiles), dim3(256), 0, nc::stream(), (float *)p[0],
+                       (unsigned long long *)p[1], (const float *)p[2], (const float4 *)p[3], (int)s[0], s[1],
+                       (int)s[2], (const float *)p[5], (const float *)p[6], slots);
+    return nc::launched("head_rows");
+}
+
+
 
 __global__ void fill_u64(unsigned long long *p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -287,6 +481,16 @@ NC_EXPORT int32_t nc_lm_head(void **p, const int64_t *s) {
     const int64_t blocks = (s[1] + 63) / 64;
     const dim3 grid((unsigned)blocks, (unsigned)s[0]);
     const int slots = s[4] ? (int)grid.x : 0;
+    // Several rows: 16 a wave once that leaves two waves a SIMD, 4 a wave down to one wave a SIMD of
+    // the one-row kernels' (which read the table anew for every row, but whose
+    // many short waves hide what a few long ones cannot). Measured on MI355X, us, one row / 4 / 16 a wave:
+    // 128 x 151936 x 896: 10160 / 924 / 579; 16: 1272 / 167 / 124; 4: 322 / 104 / 122; 500 x 4864 x 896:
+    // 718 / 113 / 100; 128 x 4864 x 896: 141 / 39 / 50; 500 x 896 x 4864: 734 / 130 / 248;
+    // 16 x 4864 x 896: 21.1 / 20.3 / 49; 8 x 8192 x 8192: 228 / 195 / 410; 33 x 896 x 896: 10.6 / 20.6 / 49; 4 x 4864 x 896: 10.8 / 20.9 / 52.
+    if (s[0] > 1 && !p[4] && ((uintptr_t)p[2] & 15) == 0) {
+        if (s[0] > 4 && (s[0] + 15) / 16 * blocks >= 2048) return launch_head_rows<16>(p, s, slots);
+        if (s[0] * blocks >= 1000) return launch_head_rows<4>(p, s, slots);
+    }
     if (s[2] == 896) {       // the model's width: the ring kernel, 24 loads (24 KB) in flight per wave
         hipLaunchKernelGGL((lm_head_ring<896, 24>), grid, dim3(64), 0, nc::stream(), (float *)p[0],
                            (unsigned long long *)p[1], (const float *)p[2], (const float4 *)p[3], s[1],
