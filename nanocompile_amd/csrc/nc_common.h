@@ -196,6 +196,10 @@ int32_t gemm_tile_info(int tile, int64_t *out);
 // attention workspace the library holds for nc_attention_decode_static
 // (nc_attention.hip); called once per device by nc_init.
 int32_t attention_scratch_init(int device);
+// matmul_i8 over several rows on the float32 matrix cores (nc_chains.hip), and whether it takes a problem.
+bool matmul_i8_rows_ok(const float *x, const int8_t *packed, int64_t M, int64_t N, int64_t K);
+int32_t matmul_i8_rows(float *y, const float *x, const int8_t *packed, const int8_t *q, const float *scales,
+                       const float *bias, const float *residual, const float *gate, int64_t M, int64_t N, int64_t K);
 // The per-token quantizer (nc_quant.hip) on M rows of K: xq, xs from x.
 int32_t quantize_token_rows(int8_t *xq, float *xs, const float *x, int M, int K);
 }  // namespace nc

@@ -659,6 +659,9 @@ NC_EXPORT int32_t nc_matmul_i8(void **p, const int64_t *s) {
     NC_REQUIRE(s[0] >= 0 && s[0] < 65536 && s[1] >= 0 && s[1] < (1 << 24) && s[2] > 0 && s[2] <= 16384,
                "nc_matmul_i8: bad shape (K at most 16384)");
     if (s[0] == 0 || s[1] == 0) return NC_OK;
+    if (nc::matmul_i8_rows_ok((const float *)p[1], (const int8_t *)p[2], s[0], s[1], s[2]))
+        return nc::matmul_i8_rows((float *)p[0], (const float *)p[1], (const int8_t *)p[2], (const int8_t *)p[3],
+                                  (const float *)p[4], (const float *)p[5], (const float *)p[6], nullptr, s[0], s[1], s[2]);
     // the model's widths, x 16-byte aligned: a chain a lane, the row staged in 16-byte pieces
     const bool whole = ((uintptr_t)p[1] & 15) == 0;
     if (whole && (s[2] == 896 || s[2] == 4864)) {
@@ -703,6 +706,9 @@ NC_EXPORT int32_t nc_matmul_i8_silu(void **p, const int64_t *s) {
                    ((uintptr_t)p[1] & 15) == 0 && p[0] != p[1],
                "nc_matmul_i8_silu: bad shape (K 896 or 4864, x 16-byte aligned, h not x)");
     if (s[0] == 0 || s[1] == 0) return NC_OK;
+    if (nc::matmul_i8_rows_ok((const float *)p[1], (const int8_t *)p[2], s[0], s[1], s[2]))
+        return nc::matmul_i8_rows((float *)p[0], (const float *)p[1], (const int8_t *)p[2], (const int8_t *)p[3],
+                                  (const float *)p[4], nullptr, nullptr, (const float *)p[5], s[0], s[1], s[2]);
     const auto kernel = s[2] == 896 ? matmul_i8_lanes<7> : matmul_i8_lanes<38>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)((s[1] + 7) / 8), (unsigned)s[0]), dim3(256), 0, nc::stream(),
                        (float *)p[0], (const float *)p[1], (const int8_t *)p[2], (const float *)p[4],

@@ -405,7 +405,7 @@ class Qwen2:
         eps = float_bits(c.rms_norm_eps)
         for i, w in enumerate(self.layers):
             kc, vc = cache.layer(i)
-            if self._fused_norm(H):                # the norm inside the projection: the same bits
+            if self._fused_norm(H, m):             # the norm inside the projection: the same bits
                 self._project_normed(w["qkv"], w["g1"], self.qkv, m, W, H, eps, bias=w["qkv_b"])
             elif self._normed_blocks(H):           # the norm inside the block quantizer: the same bits
                 hip.call("nc_quantize_blocks_normed", [self.xq, self.xsb, self.xoff, self.x, w["g1"]], [m, H, eps])
@@ -436,12 +436,13 @@ class Qwen2:
                 hip.call("nc_silu_mul", [self.h, self.gate, self.up], [m * I])
             self._project(w["down"], self.h, self.x, m, H, I, residual=self.x)
 
-    def _fused_norm(self, k: int) -> bool:
+    def _fused_norm(self, k: int, m: int) -> bool:
         """Whether int8 mode's qkv projection takes the first norm in (nc_matmul_i8_normed, the
         model's widths; the residual stream is 256-byte aligned in the arena). Only there: its
         144 workgroups repeat the norm's chain in one round, where the gate and up projections'
-        608 each would repeat it over several (measured slower)."""
-        return self.quantization == "int8" and k in (896, 4864)
+        608 each would repeat it over several (measured slower); and only for a few tokens, as
+        from 16 on the projection without the norm runs on the matrix cores (the same bits)."""
+        return self.quantization == "int8" and k in (896, 4864) and m < 16
 
     def _silu_epilogue(self, k: int) -> bool:
         """Whether the reference modes' up projection applies SwiGLU in its epilogue
