@@ -24,6 +24,7 @@
 #include "nc_common.h"
 #include "nc_attend.h"
 #include "nc_epilogue.h"
+#include "nc_exp.h"
 #include "nc_math.h"
 
 namespace {
@@ -155,7 +156,8 @@ __global__ __launch_bounds__(kThreads) void rope_append(float *__restrict__ qkv,
 // e = 0 (m_j), 1 (l_j), 2 + d (o_j[d]); jstride = the chunks of the longest
 // context of the call.
 constexpr int kWaves = 8;              // decode: waves of a chunk workgroup, one query head each
-// Prefill: 4 query rows per workgroup, one per wave. A wave attends its row's
+// Prefill on the vector ALU (attention_rows_chunks: the schedules 1 .. 4, and groups of more
+// than 64 heads): 4 query rows per workgroup, one per wave. A wave attends its row's
 // heads of the group together, up to 7 at a time (nc_attend.h's
 // chunk_scores_sq and chunk_values_n: every key or value element read from LDS
 // once for all the heads' chains, the row's queries read with scalar loads
@@ -172,7 +174,7 @@ constexpr int kWaves = 8;              // decode: waves of a chunk workgroup, on
 // query read with scalar loads (69-73 us).
 constexpr int kRowsPerBlock = 4;         // prefill: query rows (waves) a chunk workgroup, the library's choice
 // The prefill schedules a tuner may choose: schedule s (1..4) stages each
-// chunk for kScheduleRows[s - 1] rows; schedule 0 is kRowsPerBlock. Every
+// chunk for kScheduleRows[s - 1] rows; schedule 0 is attention_rows_mfma. Every
 // choice computes the same bits: a row's arithmetic does not depend on which
 // workgroup holds it.
 constexpr int kScheduleRows[4] = {2, 4, 8, 16};
@@ -259,17 +261,217 @@ __global__ __launch_bounds__(64 * ROWS) void attention_rows_chunks(
     }
 }
 
+// The same chunk results on the float32 matrix cores, for a prompt's rows. Each
+// element of v_mfma_f32_16x16x4_f32 is the chain fmaf(a[k], b[k], acc), k = 0 .. 3
+// in order (measured on gfx950, bit for bit, subnormals kept), so a score's chain
+// over d and a context element's over the keys run four steps an instruction, for 16
+// keys (or 16 d) by 16 queries, in nc_attend.h's order and with its bits.
+//
+// A workgroup (four waves) takes a chunk of one KV head and a block of R = 64 / group
+// query rows: its queries are the (row, head of the group) pairs, 16 a wave, so a group
+// of 7 fills 63 of 64 columns. Lane (c, kq) (c = lane % 16, kq = lane / 16) holds query c:
+// of S = K q its four registers a tile of 16 keys are keys 16 T + 4 r + kq (the key
+// tile's rows are taken in that order), which is just what P V's instruction for keys
+// 4 s .. 4 s + 3 (s = 4 T + r) wants from it, so the probabilities never move; l's
+// butterfly (xor 32, 16, 8, 4 of the key in registers, 2 and 1 across lanes) is the
+// wavefront sum's tree. Keys are staged with d in the order (d % 4, d / 4), values
+// transposed with the key in that order, so a lane's operands of four steps are one
+// 16-byte read.
+//
+// Masked keys have p = 0, which leaves a context chain as it is unless the value is
+// infinite or NaN: a chunk holding such a value that some row of the block must not
+// see is taken a row at a time, the masked values as zeros.
+//
+// The float32 matrix instructions and the vector ALU share their units (a loop of both
+// took the sum of their times), so the bound is 128 multiply-adds a (query, key) at the
+// 77 T/s the instructions reach alone plus the softmax's vector instructions, about as
+// much again: 2,048 rows, 50 + 45 us; measured with the combine 164 us, against 242 with
+// attention_rows_chunks (512 rows: 21.7 against 25.8). What is left there is the chunk
+// results (125 MB written and read) and the short life of a workgroup; 32 queries a wave,
+// for half the LDS reads, measured slower (177 and 25.1: fewer, longer workgroups).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef f32x4 __attribute__((aligned(8))) f32x4_at8;      // a chunk result is D + 2 floats: 8-byte aligned
+
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attention_rows_mfma(
+    float *__restrict__ part, const float *__restrict__ qkv, const float *__restrict__ kcache,
+    const float *__restrict__ vcache, int heads, int kv_heads, int past, int capacity, float scale, int i0, int rows,
+    int M, int jstride, int R, const int64_t *__restrict__ pos_ptr, int32_t *__restrict__ error) {
+    if (pos_ptr && !position_fits(pos_ptr, M, capacity, error, past)) return;
+    // The block of rows and the chunk: block z sees chunks 0 .. chunks_of(z) - 1, more the later its rows;
+    // a z of the grid holds block z's chunks, then those of the block as far from the end, together the
+    // same number for every z, so few workgroups have nothing to do (with one z a block, a causal
+    // prompt's dead half left some CUs four live workgroups and others one).
+    const int nblocks = (rows + R - 1) / R;
+    auto chunks_of = [&](int z) { return (past + i0 + min((z + 1) * R, rows) - 1) / nc::kChunk + 1; };
+    int z = blockIdx.z, j = blockIdx.x;
+    if (j >= chunks_of(z)) {
+        j -= chunks_of(z);
+        if (nblocks - 1 - z == z) return;
+        z = nblocks - 1 - z;
+        if (j >= chunks_of(z)) return;
+    }
+    const int g = blockIdx.y, t0 = j * nc::kChunk;
+    const int rb0 = z * R, r_last = min(rb0 + R, rows) - 1;
+    constexpr int KSTRIDE = D + 4, VSTRIDE = nc::kChunk + 16, STEPS = D / 4, TILES = D / 16;
+    __shared__ __align__(16) float sk[nc::kChunk * KSTRIDE], sv[D * VSTRIDE];
+    __shared__ int odd_value;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c16 = lane & 15, kq = lane >> 4;
+    const int group = heads / kv_heads, width = (heads + 2 * kv_heads) * D;
+    nc::ChunkLoad<D, 256> load;
+    load.issue(kcache + (size_t)g * capacity * D, vcache + (size_t)g * capacity * D, t0, capacity - 1);
+
+    const int qi = wave * 16 + c16, row = qi / group, r = rb0 + row, head = g * group + qi - row * group;
+    const bool valid = row < R && r < rows && past + i0 + r + 1 > t0;
+    const int n = min(nc::kChunk, past + i0 + r + 1 - t0);
+    float q[STEPS];
+    {
+        const float *src = valid ? qkv + (size_t)(i0 + r) * width + head * D : qkv;
+        // four consecutive d a load, then lanes' kq and registers' e trade places: q[4 x + y] is d = 16 x + 4 y + kq
+#pragma unroll
+        for (int x = 0; x < TILES; ++x) {
+            const float4 v = *reinterpret_cast<const float4 *>(src + 16 * x + 4 * kq);
+            const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.x), __float_as_uint(v.z), false, false);
+            const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v.y), __float_as_uint(v.w), false, false);
+            const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+            const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+            q[4 * x + 0] = __uint_as_float(lo[0]);
+            q[4 * x + 1] = __uint_as_float(lo[1]);
+            q[4 * x + 2] = __uint_as_float(hi[0]);
+            q[4 * x + 3] = __uint_as_float(hi[1]);
+        }
+    }
+    if (threadIdx.x == 0) odd_value = 0;
+    __syncthreads();
+    const int have = past + M - t0;                       // keys from it on: not yet in the cache, taken as zeros
+    {
+        typedef nc::ChunkLoad<D, 256> L;
+        float odd = 0.0f;                                 // 0 times every value: NaN where one is infinite or NaN
+#pragma unroll
+        for (int it = 0; it < L::kIters; ++it) {
+            const int u = threadIdx.x + it * 256, key = u / L::kRow4, x = u % L::kRow4;
+            if (L::kTotal % 256 == 0 || u < L::kTotal) {
+                float kx[4] = {load.k[it].x, load.k[it].y, load.k[it].z, load.k[it].w};
+                float vx[4] = {load.v[it].x, load.v[it].y, load.v[it].z, load.v[it].w};
+                if (have < nc::kChunk) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        kx[e] = key < have ? kx[e] : 0.0f;
+                        vx[e] = key < have ? vx[e] : 0.0f;
+                    }
+                }
+                // (row d = 4 x + e; the key's place is permuted by x % 4 within 16 against bank conflicts)
+                const int at = ((key & 3) * 16 + (key >> 2)) ^ (4 * (x & 3));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    sk[key * KSTRIDE + e * STEPS + x] = kx[e];
+                    sv[(4 * x + e) * VSTRIDE + at] = vx[e];
+                    odd = __builtin_fmaf(vx[e], 0.0f, odd);
+                }
+            }
+        }
+        if (odd != odd) odd_value = 1;                    // (every writer writes the same)
+    }
+    __syncthreads();
+
+    // Scores: tiles of keys some row of the block sees; the others stay masked.
+    const int seen = min(nc::kChunk, past + i0 + r_last + 1 - t0), tiles = (seen + 15) / 16;
+    f32x4 s[4];
+#pragma unroll
+    for (int T = 0; T < 4; ++T) {
+        s[T] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (T < tiles) {
+            const float *krow = sk + (16 * T + 4 * (c16 & 3) + (c16 >> 2)) * KSTRIDE + kq * STEPS;
+#pragma unroll
+            for (int x = 0; x < STEPS / 4; ++x) {
+                const f32x4 k4 = *reinterpret_cast<const f32x4 *>(krow + 4 * x);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s[T] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], q[4 * x + e], s[T], 0, 0, 0);
+            }
+        }
+    }
+    const bool partial = past + i0 + rb0 + 1 - t0 < nc::kChunk;       // some row does not see the whole chunk
+    float l, m = -__builtin_inff();
+    {
+        // The maximum of the scores that are not NaN: with a NaN among them the chunk's l and o are NaN
+        // either way, and so is what the combine makes of them.
+#pragma unroll
+        for (int T = 0; T < 4; ++T)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s[T][e] = __builtin_fmaf(s[T][e], scale, 0.0f);      // * scale, + 0 of the mask
+                if (partial) s[T][e] = 16 * T + 4 * e + kq < n ? s[T][e] : -__builtin_inff();
+                m = __builtin_fmaxf(m, s[T][e]);
+            }
+        m = nc::butterfly_step<32>(m, [](float a, float b) { return __builtin_fmaxf(a, b); });
+        m = nc::butterfly_step<16>(m, [](float a, float b) { return __builtin_fmaxf(a, b); });
+#pragma unroll
+        for (int T = 0; T < 4; ++T)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[T][e] = nc_expf_upto100(__fsub_rn(s[T][e], m));
+        // the wavefront sum's tree over the key's bits 5, 4 (T), 3, 2 (e), 1, 0 (kq)
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = __fadd_rn(__fadd_rn(s[0][e], s[2][e]), __fadd_rn(s[1][e], s[3][e]));
+        float sum = __fadd_rn(__fadd_rn(v[0], v[2]), __fadd_rn(v[1], v[3]));
+        sum = nc::butterfly_step<32>(sum, [](float a, float b) { return __fadd_rn(a, b); });
+        sum = nc::butterfly_step<16>(sum, [](float a, float b) { return __fadd_rn(a, b); });
+        l = sum;
+    }
+
+    // Context: keys in order, four an instruction; `limit`: values of keys from it on taken as zeros.
+    f32x4 o[TILES];
+    auto context = [&](int limit) {
+#pragma unroll
+        for (int dt = 0; dt < TILES; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int T = 0; T < 4; ++T) {
+            if (T < tiles) {
+#pragma unroll
+                for (int dt = 0; dt < TILES; ++dt) {
+                    const int d = 16 * dt + c16;
+                    f32x4 v4 = *reinterpret_cast<const f32x4 *>(sv + d * VSTRIDE +
+                                                                ((kq * 16 + 4 * T) ^ (4 * ((d >> 2) & 3))));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (16 * T + 4 * e + kq >= limit) v4[e] = 0.0f;
+                        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[e], s[T][e], o[dt], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    };
+    auto keep = [&]() {
+        if (!valid) return;
+        float *dst = chunk_result(part, head, rows, r, jstride, j, D);
+        if (kq == 0) *reinterpret_cast<f32x2 *>(dst) = f32x2{m, l};
+#pragma unroll
+        for (int dt = 0; dt < TILES; ++dt) *reinterpret_cast<f32x4_at8 *>(dst + 2 + 16 * dt + 4 * kq) = o[dt];
+    };
+    if (odd_value && partial) {
+        for (int i = rb0; i <= r_last; ++i) {             // (uniform over the workgroup)
+            context(past + i0 + i + 1 - t0);
+            if (r == i) keep();
+        }
+        return;
+    }
+    context(nc::kChunk);
+    keep();
+}
+
 // The combine of one query's chunk results: grid (heads, rows), one wave.
 // Row r of the slab is query row i0 + r at position past + i0 + r. The first
-// 64 * BATCH floats of the row's results (BATCH = 8: up to 7 chunks, 448 keys,
-// at D = 64; 16: up to 15 chunks, 960 keys) are loaded before the position is
-// read, all in flight at once.
-template <int D, int BATCH>
+// 512 floats of the row's results (up to 7 chunks, 448 keys, at D = 64) are loaded
+// before the position is read, all in flight at once.
+template <int D>
 __global__ __launch_bounds__(64) void attention_combine(float *__restrict__ ctx, const float *__restrict__ part,
                                                         int heads, int past, int capacity, int i0, int rows, int M,
                                                         int jstride, const int64_t *__restrict__ pos_ptr) {
     extern __shared__ __align__(16) float results[];     // [J][D + 2]
-    constexpr int kBatch = BATCH;                        // independent loads a lane keeps in flight
+    constexpr int kBatch = 8;                            // independent loads a lane keeps in flight
     const int h = blockIdx.x, r = blockIdx.y, lane = threadIdx.x;
     const float *src = chunk_result(part, h, rows, r, jstride, 0, D);
     const int all = jstride * (D + 2);
@@ -306,46 +508,119 @@ __global__ __launch_bounds__(64) void attention_combine(float *__restrict__ ctx,
     if (lane < D) ctx[(size_t)(i0 + r) * heads * D + h * D + lane] = out;
 }
 
-// The combine of a whole query row, one wave per head (grid rows, heads x 64
-// threads), then the row's per-token int8 quantization (nc_quant.hip's
-// quantize_token: the maximum of |ctx| over the row, its scale, each value
-// quantized) in the same launch: ctx, xq and xs with the bits of a combine
-// followed by nc_quantize_token_i8.
-template <int D, int BATCH>
-__global__ __launch_bounds__(1024) void attention_combine_quant(float *__restrict__ ctx, int8_t *__restrict__ xq,
-                                                                float *__restrict__ xs, const float *__restrict__ part,
-                                                                int heads, int past, int capacity, int i0, int rows,
-                                                                int M, int jstride, const int64_t *__restrict__ pos_ptr) {
+// The combine of one query over a long context: grid (heads, rows), four waves that bring
+// the chunk results to LDS together (16 loads a thread in flight, 62 chunks at D = 64),
+// then one wave in combine_chunks' order.
+template <int D>
+__global__ __launch_bounds__(256) void attention_combine_wide(float *__restrict__ ctx, const float *__restrict__ part,
+                                                              int heads, int past, int capacity, int i0, int rows,
+                                                              int M, int jstride, const int64_t *__restrict__ pos_ptr) {
+    extern __shared__ __align__(16) float results[];     // [J][D + 2]
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    constexpr int kBatch = 8;
+    const int h = blockIdx.x, r = blockIdx.y;
+    // D + 2 is even: a query's results are whole pairs, 8-byte aligned
+    const f32x2 *src = reinterpret_cast<const f32x2 *>(chunk_result(part, h, rows, r, jstride, 0, D));
+    const int all = jstride * (D + 2) / 2;
+    f32x2 v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) v[u] = src[min((int)threadIdx.x + 256 * u, all - 1)];
     if (pos_ptr) {
         const int64_t p = *pos_ptr;
         if (p < 0 || p + M > capacity) return;            // the chunk kernel reported it
         past = (int)p;
     }
-    extern __shared__ __align__(16) float results_all[];   // [heads][jstride][D + 2]
-    __shared__ float maxima[16];
-    const int r = blockIdx.x, lane = threadIdx.x & 63, h = threadIdx.x >> 6;
     const int J = (past + i0 + r + 1 + nc::kChunk - 1) / nc::kChunk;
-    float *results = results_all + (size_t)h * jstride * (D + 2);
-    const float *src = chunk_result(part, h, rows, r, jstride, 0, D);
-    const int total = J * (D + 2);
-    constexpr int kBatch = BATCH;                        // loads a lane keeps in flight
-    for (int base = 0; base < total; base += 64 * kBatch) {
-        float v[kBatch];
+    const int total = J * (D + 2) / 2;
+    f32x2 *dst = reinterpret_cast<f32x2 *>(results);
+    for (int base = 0; base < total; base += 256 * kBatch) {
+        if (base > 0) {
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-            const int at = base + lane + 64 * u;
-            v[u] = at < total ? src[at] : 0.0f;
+            for (int u = 0; u < kBatch; ++u) v[u] = src[min(base + (int)threadIdx.x + 256 * u, total - 1)];
         }
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
-            const int at = base + lane + 64 * u;
-            if (at < total) results[at] = v[u];
+            const int at = base + threadIdx.x + 256 * u;
+            if (at < total) dst[at] = v[u];
         }
     }
-    const float out = nc::combine_chunks(J, lane < D ? lane : 0,
-                                         [&](int c, int k) { return results[c * (D + 2) + k]; });
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x, dl = lane < D ? lane : 0;
+    float m = -__builtin_inff();
+    for (int j = lane; j < J; j += 64) m = nc::nan_max(m, results[j * (D + 2)]);
+    m = nc::wave_max_f32(m);
+    float L = 0.0f, O = 0.0f;
+    for (int j0 = 0; j0 < J; j0 += 64) {
+        const float *mine = results + min(j0 + lane, J - 1) * (D + 2);
+        const float w = nc_expf_upto100(__fsub_rn(mine[0], m)), l = mine[1];
+        const int end = min(64, J - j0);
+        for (int j = 0; j < end; j += 8) {
+            float o[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) o[u] = results[min(j0 + j + u, J - 1) * (D + 2) + 2 + dl];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (j + u >= end) break;
+                const float wj = nc::lane_value(w, j + u);
+                L = __fadd_rn(L, __fmul_rn(nc::lane_value(l, j + u), wj));
+                O = __fadd_rn(O, __fmul_rn(o[u], wj));
+            }
+        }
+    }
+    if (lane < D) ctx[(size_t)(i0 + r) * heads * D + h * D + lane] = nc::div_rn(O, L);
+}
+
+// The combine of a whole query row of at most 64 chunks: one wave per head (at most 16),
+// then the row's per-token int8 quantization (nc_quant.hip's quantize_token: the maximum of
+// |ctx| over the row, its scale, each value quantized) in the same launch when xq is given:
+// ctx, xq and xs with the bits of a combine followed by nc_quantize_token_i8. Lane j holds
+// chunk j's m, l and weight; the context values come straight from memory, a row of D floats
+// a load, a batch of them in flight from the start.
+template <int D>
+__global__ __launch_bounds__(1024) void attention_combine_rows(float *__restrict__ ctx, int8_t *__restrict__ xq,
+                                                               float *__restrict__ xs, const float *__restrict__ part,
+                                                               int heads, int past, int capacity, int i0, int rows,
+                                                               int M, int jstride, const int64_t *__restrict__ pos_ptr) {
+    if (pos_ptr) {
+        const int64_t p = *pos_ptr;
+        if (p < 0 || p + M > capacity) return;            // the chunk kernel reported it
+        past = (int)p;
+    }
+    __shared__ float maxima[16];
+    const int r = blockIdx.x, lane = threadIdx.x & 63, h = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int J = (past + i0 + r + 1 + nc::kChunk - 1) / nc::kChunk;
+    const float *src = chunk_result(part, h, rows, r, jstride, 0, D);
+    const float *o = src + 2 + (lane < D ? lane : 0);
+    constexpr int BATCH = 8;           // (16 and 32 measured no faster at 512 and 2,048 rows)
+    float v[BATCH];
+    auto fetch = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) v[u] = o[min(j0 + u, J - 1) * (D + 2)];
+    };
+    fetch(0);
+    const float *mine = src + min(lane, J - 1) * (D + 2);
+    const float mj = mine[0], lj = mine[1], m = nc::wave_max_f32(mj);       // (the last chunk's again past it)
+    const float w = nc_expf_upto100(__fsub_rn(mj, m));
+    float L = 0.0f, O = 0.0f;
+    for (int j0 = 0; j0 < J; j0 += BATCH) {
+        float now[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) now[u] = v[u];
+        if (j0 + BATCH < J) fetch(j0 + BATCH);
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            if (j0 + u < J) {
+                const float wj = nc::lane_value(w, j0 + u);
+                L = __fadd_rn(L, __fmul_rn(nc::lane_value(lj, j0 + u), wj));
+                O = __fadd_rn(O, __fmul_rn(now[u], wj));
+            }
+        }
+    }
+    const float out = nc::div_rn(O, L);
     const size_t at = (size_t)(i0 + r) * heads * D + h * D + lane;
     if (lane < D) ctx[at] = out;
+    if (!xq) return;
     const float mag = nc::wave_max_f32(lane < D ? fabsf(out) : 0.0f);
     if (lane == 0) maxima[h] = mag;
     __syncthreads();
@@ -506,12 +781,12 @@ namespace {
 
 // LDS of a combine: J chunk results of D + 2 floats, 67.6 KB at 16384 keys and
 // D = 64, past the 64 KB a launch gets without asking.
-template <int D, int BATCH>
-int32_t launch_combine_batch(float *ctx, const float *part, int64_t heads, int64_t past, int64_t cap, int64_t i0,
-                             int64_t rows, int64_t M, int64_t jstride, const int64_t *pos) {
-    static bool raised = false;
+template <typename K>
+int32_t launch_combine_kernel(K kernel, bool &raised, unsigned threads, int D, float *ctx, const float *part,
+                              int64_t heads, int64_t past, int64_t cap, int64_t i0, int64_t rows, int64_t M,
+                              int64_t jstride, const int64_t *pos) {
     if (!raised) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_combine<D, BATCH>),
+        if (hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024) != hipSuccess) {
             nc::set_message("attention: could not raise the LDS limit of the combine");
             return NC_LAUNCH_FAILED;
@@ -519,37 +794,36 @@ int32_t launch_combine_batch(float *ctx, const float *part, int64_t heads, int64
         raised = true;
     }
     const size_t lds = (size_t)jstride * (D + 2) * sizeof(float);
-    hipLaunchKernelGGL((attention_combine<D, BATCH>), dim3((unsigned)heads, (unsigned)rows), dim3(64), lds,
+    hipLaunchKernelGGL(kernel, dim3((unsigned)heads, (unsigned)rows), dim3(threads), lds,
                        nc::stream(), ctx, part, (int)heads, (int)past, (int)cap, (int)i0, (int)rows, (int)M,
                        (int)jstride, pos);
     return nc::launched("attention_combine");
 }
 
-// The first batch of loads sized to the chunk results a row can have.
+// One wave while a row's results are one batch of its loads (up to 7 chunks at D = 64), else four.
 template <int D>
 int32_t launch_combine(float *ctx, const float *part, int64_t heads, int64_t past, int64_t cap, int64_t i0,
                        int64_t rows, int64_t M, int64_t jstride, const int64_t *pos) {
+    static bool raised[2] = {};
     if (jstride * (D + 2) <= 64 * 8)
-        return launch_combine_batch<D, 8>(ctx, part, heads, past, cap, i0, rows, M, jstride, pos);
-    return launch_combine_batch<D, 16>(ctx, part, heads, past, cap, i0, rows, M, jstride, pos);
+        return launch_combine_kernel(&attention_combine<D>, raised[0], 64, D, ctx, part, heads, past, cap, i0, rows, M,
+                                     jstride, pos);
+    return launch_combine_kernel(&attention_combine_wide<D>, raised[1], 256, D, ctx, part, heads, past, cap, i0, rows,
+                                 M, jstride, pos);
 }
 
-// A head's chunk results in one batch of loads up to 9 chunks at D = 64 (576
-// floats: a 512-token prompt's 8 chunks in one memory round trip), else in
-// batches of 16 loads a lane.
 template <int D>
-int32_t launch_combine_quant(void **p, const float *part, int64_t heads, int64_t past, int64_t cap, int64_t i0,
-                             int64_t rows, int64_t M, int64_t jstride, const int64_t *pos) {
-    const size_t lds = (size_t)heads * jstride * (D + 2) * sizeof(float);
-    auto kernel = jstride * (D + 2) <= 64 * 9 ? attention_combine_quant<D, 9> : attention_combine_quant<D, 16>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3((unsigned)(64 * heads)), lds, nc::stream(), (float *)p[0],
-                       (int8_t *)p[6], (float *)p[7], part, (int)heads, (int)past, (int)cap, (int)i0, (int)rows,
-                       (int)M, (int)jstride, pos);
-    return nc::launched("attention_combine_quant");
+int32_t launch_combine_rows(void **p, bool quantize, const float *part, int64_t heads, int64_t past, int64_t cap,
+                            int64_t i0, int64_t rows, int64_t M, int64_t jstride, const int64_t *pos) {
+    hipLaunchKernelGGL(attention_combine_rows<D>, dim3((unsigned)rows), dim3((unsigned)(64 * heads)), 0, nc::stream(), (float *)p[0],
+                       quantize ? (int8_t *)p[6] : nullptr, (float *)p[7], part, (int)heads, (int)past, (int)cap,
+                       (int)i0, (int)rows, (int)M, (int)jstride, pos);
+    return nc::launched("attention_combine_rows");
 }
 
 // Query rows in slabs whose chunk results fit the workspace; each slab is a
-// chunk launch and a combine launch.
+// chunk launch and a combine launch. ROWS 0: the matrix-core chunk kernel, else
+// attention_rows_chunks with ROWS rows a workgroup.
 template <int D, int ROWS>
 int32_t launch_prefill(void **p, int64_t M, int64_t heads, int64_t kv, int64_t past, int64_t cap, float scale,
                        const int64_t *pos, float *work, int64_t work_bytes) {
@@ -559,24 +833,41 @@ int32_t launch_prefill(void **p, int64_t M, int64_t heads, int64_t kv, int64_t p
     NC_REQUIRE(slab >= 1, "nc_attention: the workspace is smaller than one query row's chunk results "
                           "(heads * ceil(keys / 64) * (head_dim + 2) floats)");
     // with xq and xs, the per-token int8 of ctx too: in the combine's own launch
-    // while a row's chunk results fit its workgroup's LDS, else after
+    // while a workgroup's waves hold a row's heads, else after
     const bool quantize = p[6] && p[7];
-    const bool fused = quantize && heads <= 16 && heads * jstride * (D + 2) * (int64_t)sizeof(float) <= 64 * 1024;
-    if (slab < M && slab >= ROWS) slab -= slab % ROWS;
+    const bool whole_rows = heads <= 16 && jstride <= 64;
+    const bool fused = quantize && whole_rows;
+    const int64_t unit = ROWS ? ROWS : 64 / (heads / kv);     // rows a workgroup takes
+    if (slab < M && slab >= unit) slab -= slab % unit;
     const int64_t host_past = pos ? 0 : past;
     for (int64_t i0 = 0; i0 < M; i0 += slab) {
         const int64_t rows = std::min(slab, M - i0);
-        const int64_t chunks = pos ? jstride : (past + i0 + rows + nc::kChunk - 1) / nc::kChunk;
-        hipLaunchKernelGGL((attention_rows_chunks<D, ROWS>),
-                           dim3((unsigned)chunks, (unsigned)kv, (unsigned)((rows + ROWS - 1) / ROWS)),
-                           dim3(64 * ROWS), 0, nc::stream(), work, (const float *)p[1], (const float *)p[2],
-                           (const float *)p[3], (int)heads, (int)kv, (int)host_past, (int)cap, scale, (int)i0,
-                           (int)rows, (int)M, (int)jstride, pos, nc::error_word());
+        if (ROWS == 0) {
+            const int64_t R = 64 / (heads / kv), blocks = (rows + R - 1) / R;
+            auto chunks_of = [&](int64_t z) { return (past + i0 + std::min((z + 1) * R, rows) - 1) / nc::kChunk + 1; };
+            int64_t most = blocks > 1 ? 2 * jstride : jstride;   // chunks of a z of the grid: one block's, or two's
+            if (!pos) {
+                most = 0;
+                for (int64_t z = 0; z < (blocks + 1) / 2; ++z)
+                    most = std::max(most, chunks_of(z) + (blocks - 1 - z == z ? 0 : chunks_of(blocks - 1 - z)));
+            }
+            hipLaunchKernelGGL(attention_rows_mfma<D>, dim3((unsigned)most, (unsigned)kv, (unsigned)((blocks + 1) / 2)),
+                               dim3(256), 0, nc::stream(), work, (const float *)p[1], (const float *)p[2],
+                               (const float *)p[3], (int)heads, (int)kv, (int)host_past, (int)cap, scale, (int)i0,
+                               (int)rows, (int)M, (int)jstride, (int)R, pos, nc::error_word());
+        } else {
+            constexpr int WAVES = ROWS ? ROWS : 1;
+            const int64_t chunks = pos ? jstride : (past + i0 + rows + nc::kChunk - 1) / nc::kChunk;
+            hipLaunchKernelGGL((attention_rows_chunks<D, WAVES>),
+                               dim3((unsigned)chunks, (unsigned)kv, (unsigned)((rows + WAVES - 1) / WAVES)),
+                               dim3(64 * WAVES), 0, nc::stream(), work, (const float *)p[1], (const float *)p[2],
+                               (const float *)p[3], (int)heads, (int)kv, (int)host_past, (int)cap, scale, (int)i0,
+                               (int)rows, (int)M, (int)jstride, pos, nc::error_word());
+        }
         int32_t rc = nc::launched("attention_rows_chunks");
-        if (rc == NC_OK && fused)
-            rc = launch_combine_quant<D>(p, work, heads, host_past, cap, i0, rows, M, jstride, pos);
-        else if (rc == NC_OK)
-            rc = launch_combine<D>((float *)p[0], work, heads, host_past, cap, i0, rows, M, jstride, pos);
+        if (rc == NC_OK)
+            rc = whole_rows ? launch_combine_rows<D>(p, fused, work, heads, host_past, cap, i0, rows, M, jstride, pos)
+                            : launch_combine<D>((float *)p[0], work, heads, host_past, cap, i0, rows, M, jstride, pos);
         if (rc != NC_OK) return rc;
     }
     if (quantize && !fused)        // ctx whole first: the per-token scale spans every head of a row
@@ -623,13 +914,15 @@ NC_EXPORT int32_t nc_attention(void **p, const int64_t *s) {
     if (M == 0) return NC_OK;
     const float scale = nc::bits_to_float(s[6]);
     float *work = (float *)p[5];
-    const int rows = schedule == 0 ? kRowsPerBlock : kScheduleRows[schedule - 1];
+    // schedule 0: the matrix cores while a KV head's group of query heads fits a workgroup's 64 columns
+    const int rows = schedule ? kScheduleRows[schedule - 1] : heads / kv <= 64 ? 0 : kRowsPerBlock;
 #define NC_PREFILL(R)                                                                             \
     if (rows == R) {                                                                              \
         if (D == 64) return launch_prefill<64, R>(p, M, heads, kv, past, cap, scale, pos, work, work_bytes); \
         if (D == 32) return launch_prefill<32, R>(p, M, heads, kv, past, cap, scale, pos, work, work_bytes); \
         return launch_prefill<16, R>(p, M, heads, kv, past, cap, scale, pos, work, work_bytes);    \
     }
+    NC_PREFILL(0)
     NC_PREFILL(2)
     NC_PREFILL(4)
     NC_PREFILL(8)
