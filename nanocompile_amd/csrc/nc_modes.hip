@@ -20,6 +20,8 @@
 //     dwords w[128*k0 + 32c + 4l .. +3], c = 0..3: again 128 contiguous bytes.
 // Elements past the last whole 32-block (or 128-block) are read from the
 // plain row-major weights, in the reference's order.
+#include <type_traits>
+
 #include "nc_common.h"
 #include "nc_epilogue.h"
 #include "nc_math.h"
@@ -327,6 +329,40 @@ __device__ __forceinline__ void block32(float v, int lane, int8_t *q_out, float 
     }
 }
 
+// One block of 32 on 8 lanes, lane `lane` (0 .. 7) holding elements 4 lane .. + 3: block32's
+// maximum, values, scale and term with 3 exchanges instead of 5, on DPP, and 4-byte stores.
+__device__ __forceinline__ void block32x4(const float (&v)[4], int lane, int8_t *q_out, float *scale_out,
+                                          float *term_out) {
+    float mag = fabsf(v[0]);
+#pragma unroll
+    for (int i = 1; i < 4; ++i) mag = nc::nan_max(mag, fabsf(v[i]));
+    auto level = [&](auto off) {
+        constexpr int OFF = decltype(off)::value;
+        const float other = nc::xor_partner<OFF>(mag);
+        const bool left = (lane & OFF) == 0;
+        mag = nc::nan_max(left ? mag : other, left ? other : mag);
+    };
+    level(std::integral_constant<int, 1>{});
+    level(std::integral_constant<int, 2>{});
+    level(std::integral_constant<int, 4>{});
+    mag = nc::nan_max(0.0f, mag);
+    const float scale = nc::token_scale(mag);
+    int32_t sum = 0;
+    uint32_t packed = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int8_t qv = nc::quantize_value(v[i], scale);
+        packed |= (uint32_t)(uint8_t)qv << (8 * i);
+        sum += qv;
+    }
+    *reinterpret_cast<uint32_t *>(q_out + 4 * lane) = packed;
+    sum = nc::group_sum_i32<8>(sum);
+    if (lane == 0) {
+        *scale_out = scale;
+        *term_out = __fmul_rn((float)sum, scale);
+    }
+}
+
 // rms_norm_index_order of a row of K <= 1024 (a multiple of 64), then quantize_blocks of the
 // normalized row with blocks of 32, in one workgroup: the norm's bits (the sum of squares in
 // index order in thread 0, then (x * (1 / sqrt(ss / K + eps))) * gamma) and the quantizer's.
@@ -386,11 +422,20 @@ __global__ __launch_bounds__(256) void quantize_blocks_normed(int8_t *__restrict
 // order, of f32(sum of the block's xq) * scale.
 __global__ __launch_bounds__(256) void quantize_blocks(int8_t *__restrict__ xq, float *__restrict__ xs,
                                                        float *__restrict__ offset, const float *__restrict__ x, int K,
-                                                       int block) {
+                                                       int block, bool quads) {
     extern __shared__ float terms[];                              // one per block
     const int m = blockIdx.x, nb = K / block;
     const float *row = x + (size_t)m * K;
-    if (block == 32) {
+    if (block == 32 && quads) {
+        // four elements a lane: 32 blocks a round, a round's loads a round ahead
+        const int lane = threadIdx.x & 7, group = threadIdx.x >> 3;
+        float4 next = *reinterpret_cast<const float4 *>(row + (size_t)min(group, nb - 1) * 32 + 4 * lane);
+        for (int b = group; b < nb; b += 32) {
+            const float v[4] = {next.x, next.y, next.z, next.w};
+            next = *reinterpret_cast<const float4 *>(row + (size_t)min(b + 32, nb - 1) * 32 + 4 * lane);
+            block32x4(v, lane, xq + (size_t)m * K + (size_t)b * 32, xs + (size_t)m * nb + b, terms + b);
+        }
+    } else if (block == 32) {
         // a block of 32 on 32 lanes, an element a lane. The chain's maximum, mag = nan_max(mag,
         // |v_i|) from 0 in index order, as an ordered tree: its step is associative (a NaN on
         // the right wins, else one on the left, else the leftmost maximum), so lanes combined
@@ -727,6 +772,10 @@ NC_EXPORT int32_t nc_matmul_i8_vnni(void **p, const int64_t *s) {
                    (block & (block - 1)) == 0 && K % block == 0,
                "nc_matmul_i8_vnni: bad shape (block a power of two >= 32 dividing K)");
     if (M == 0 || N == 0) return NC_OK;
+    if (nc::matmul_i8_vnni_rows_ok((const int8_t *)p[1], (const int8_t *)p[4], (const int8_t *)p[5], M, N))
+        return nc::matmul_i8_vnni_rows((float *)p[0], (const int8_t *)p[1], (const float *)p[2], (const float *)p[3],
+                                       (const int8_t *)p[4], (const int8_t *)p[5], (const float *)p[6],
+                                       (const float *)p[7], (const float *)p[8], nullptr, M, N, K, block);
     // the model's widths, xq 16-byte aligned: a chain a lane, the row staged in 16-byte pieces
     if (((uintptr_t)p[1] & 15) == 0 && (K == 896 || K == 4864)) {
         const auto kernel = K == 896 ? matmul_i8_vnni_lanes<7> : matmul_i8_vnni_lanes<38>;
@@ -755,6 +804,10 @@ NC_EXPORT int32_t nc_matmul_i8_vnni_silu(void **p, const int64_t *s) {
                    (block & (block - 1)) == 0 && K % block == 0 && ((uintptr_t)p[1] & 15) == 0,
                "nc_matmul_i8_vnni_silu: bad shape (K 896 or 4864, block a power of two >= 32 dividing K)");
     if (M == 0 || N == 0) return NC_OK;
+    if (nc::matmul_i8_vnni_rows_ok((const int8_t *)p[1], (const int8_t *)p[4], (const int8_t *)p[5], M, N))
+        return nc::matmul_i8_vnni_rows((float *)p[0], (const int8_t *)p[1], (const float *)p[2], (const float *)p[3],
+                                       (const int8_t *)p[4], (const int8_t *)p[5], (const float *)p[6], nullptr, nullptr,
+                                       (const float *)p[7], M, N, K, block);
     const auto kernel = K == 896 ? matmul_i8_vnni_lanes<7> : matmul_i8_vnni_lanes<38>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)((N + 7) / 8), (unsigned)M), dim3(256), 0, nc::stream(),
                        (float *)p[0], (const int8_t *)p[1], (const float *)p[2], (const float *)p[3],
@@ -784,6 +837,6 @@ NC_EXPORT int32_t nc_quantize_blocks(void **p, const int64_t *s) {
     if (s[0] == 0) return NC_OK;
     hipLaunchKernelGGL(quantize_blocks, dim3((unsigned)s[0]), dim3(256), (size_t)(s[1] / s[2]) * sizeof(float),
                        nc::stream(), (int8_t *)p[0], (float *)p[1], (float *)p[2], (const float *)p[3], (int)s[1],
-                       (int)s[2]);
+                       (int)s[2], ((uintptr_t)p[3] & 15) == 0 && ((uintptr_t)p[0] & 3) == 0);
     return nc::launched("quantize_blocks");
 }

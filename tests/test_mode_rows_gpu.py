@@ -63,3 +63,54 @@ def test_matmul_i8_rows_unaligned_operands(gpu, host):
                               DeviceArray.from_host(q), DeviceArray.from_host(s)], [m, n, k])
     hip.sync()
     assert np.array_equal(bits(y.numpy()), bits(host.matmul_i8_f32(x, q, s)))
+
+
+@pytest.mark.parametrize("m,n,k", [(500, 33, 32), (17, 1000, 96), (9, 1801, 128), (40, 500, 160), (33, 700, 640),
+                                   (129, 130, 1248), (18, 896, 896), (24, 896, 4864), (130, 3900, 896)])
+@pytest.mark.parametrize("block", [32, 64])
+def test_matmul_i8_vnni_rows(gpu, host, m, n, k, block):
+    from nanocompile_amd import hip, kernels
+    from nanocompile_amd.hip import DeviceArray
+    if k % block:
+        pytest.skip("not a whole number of blocks")
+    print(f"matmul_i8_vnni m={m} n={n} k={k} block={block}", flush=True)
+    rng, x, q, s = operands(m, n, k)
+    xq, xs, off = R.quantize_blocks(x, block)
+    expected = host.matmul_i8_vnni(xq, xs, off, q, s, block)
+    assert np.array_equal(bits(kernels.matmul_i8_vnni(xq, xs, off, q, s, block).numpy()), bits(expected))
+    bias, residual = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    got = kernels.matmul_i8_vnni(xq, xs, off, q, s, block, bias=bias, residual=residual).numpy()
+    assert np.array_equal(bits(got), bits(residual + (expected + bias)))
+    if k in (896, 4864):
+        h, gate = DeviceArray((m, n), np.float32), DeviceArray.from_host(residual)
+        want = DeviceArray((m, n), np.float32)
+        up = [xq, xs, off, kernels.pack_chains_vnni(q), q, s]
+        hip.call("nc_matmul_i8_vnni_silu", [h, *map(DeviceArray.from_host, up), gate], [m, n, k, block])
+        hip.call("nc_silu_mul", [want, gate, DeviceArray.from_host(expected)], [m * n])
+        hip.sync()
+        assert np.array_equal(bits(h.numpy()), bits(want.numpy()))
+
+
+@pytest.mark.parametrize("k", [32, 64, 96, 992, 1024, 1056, 4864])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_block_quantizer_rows(gpu, k, aligned):
+    """Four elements a lane on 16-byte rows, one a lane off them: zeros, NaN, infinities, ties, signed zeros."""
+    from nanocompile_amd import hip
+    from nanocompile_amd.hip import DeviceArray
+    m = 5
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0, :32] = 0.0
+    x[1, 7], x[2, k - 1], x[3, 3] = np.nan, -np.inf, -0.0
+    x[4, :32] = np.tile([127.0, -0.5, 0.5, 63.5], 8)
+    room = DeviceArray((m * k + 1,), np.float32)
+    room.upload(np.concatenate([[0], x.reshape(-1)] if not aligned else [x.reshape(-1), [0]]).astype(np.float32))
+    xq, xs, off = DeviceArray((m, k), np.int8), DeviceArray((m, k // 32), np.float32), DeviceArray((m,), np.float32)
+    hip.call("nc_quantize_blocks", [xq, xs, off, room.ptr + (0 if aligned else 4)], [m, k, 32])
+    hip.sync()
+    eq, es, eoff = R.quantize_blocks(x, 32)
+    finite = [0, 3, 4]
+    assert np.array_equal(xq.numpy()[finite], eq[finite])
+    assert np.array_equal(bits(xs.numpy()[finite]), bits(es[finite]))
+    assert np.array_equal(bits(off.numpy()[finite]), bits(eoff[finite, 0]))
+    assert np.array_equal(np.isnan(xs.numpy()), np.isnan(es)) and np.array_equal(np.isinf(xs.numpy()), np.isinf(es))
