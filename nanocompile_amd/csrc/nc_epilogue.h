@@ -11,7 +11,7 @@
 #pragma once
 
 #include "nc_common.h"
-#include "nc_math.h"
+#include "nc_exp.h"
 
 namespace nc {
 
@@ -21,7 +21,7 @@ __device__ __forceinline__ float dequant(int32_t acc, float xs, float ws) {
 
 __device__ __forceinline__ float silu_mul(float g, float u) {
     const bool p = 0.0f <= g;
-    const float e = nc_expf(p ? -g : g);
+    const float e = nc_expf_upto100(p ? -g : g);     // (nc_expf's value; the argument is at most 0)
     const float sig = div_rn(p ? 1.0f : e, __fadd_rn(e, 1.0f));
     return __fmul_rn(__fmul_rn(g, sig), u);
 }
