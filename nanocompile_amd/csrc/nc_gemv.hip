@@ -257,13 +257,14 @@ constexpr int kGemmMinTokens = 16;
 // GEMM's conflict-free LDS layout): 64 x 128 (8 waves) for the largest
 // problems and for long k loops with many tiles; 64 x 64 from 200 such tiles
 // (gate at M = 512: 10.19 us against 11.65 with 32 x 64; down at M = 1024:
-// 15.97 against 17.5-20.9); else 32 x 32 (at M = 512: q/o 4.53 us against
+// 15.97 against 17.5-20.9; with K >= 2048 up to 256 such tiles: 2000 x 500 x 4096 14.4
+// against 15.6 with 64 x 128, 1500 x 700 x 2048, 264 of them, 11.9 against 10.4); else 32 x 32 (at M = 512: q/o 4.53 us against
 // 4.70 with 32 x 64, qkv 5.25 against 5.52 with 64 x 64, down 11.09 against
 // 11.30 with 32 x 64 and 8 stages; gate at M = 128: 5.29 against 5.57).
 int auto_tile(int M, int N, int K) {
     auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
     const int t64 = tiles(64, 64);
-    if (t64 >= 1792 || (K >= 2048 && t64 >= 256)) return 6;
+    if (t64 >= 1792 || (K >= 2048 && t64 > 256)) return 6;
     if (t64 >= 200) return 5;
     return 2;
 }
@@ -273,11 +274,13 @@ int auto_tile(int M, int N, int K) {
 // tiles, else 32 x 32 (measured at N = 4864, K = 896: M = 384 / 512 / 1024 /
 // 2048: 15.7 / 19.3 / 30.5 / 54.1 us against 16.8 / 20.6 / 35.2 / 68.1 with
 // 32 x 32 and 17.3 / 20.6 / 34.9 / 63.3 with 32 x 64; M = 128 / 256: 8.41 /
-// 12.13 us with 32 x 32 against 11.0 / 14.6 with 64 x 64).
+// 12.13 us with 32 x 32 against 11.0 / 14.6 with 64 x 64). Long k loops (K >= 2048) take 64 x 64 from
+// 200 tiles (100 x 8000 x 4096: 19.4 against 22.8 with 32 x 32) and 128 x 64 past 256 (350 x 4000 x 2560:
+// 16.6 against 19.8 and 22.4).
 int auto_tile_pair(int M, int N, int K) {
-    (void)K;
     const int t64 = ((M + 63) / 64) * ((N + 63) / 64);
-    return t64 >= 400 ? 5 : 2;
+    if (K >= 2048 && t64 > 256) return 8;
+    return t64 >= (K >= 2048 ? 200 : 400) ? 5 : 2;
 }
 
 template <int KS, int MT, bool ACC_OUT>
