@@ -14,6 +14,7 @@
 //   the LM head as a 64-bit atomic maximum of (ordered value bits, ~index), so
 //   ties go to the smallest index whatever order the waves finish in.
 #include "nc_common.h"
+#include "nc_rules.h"
 
 namespace {
 
@@ -254,11 +255,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
     const int64_t blk = (int64_t)(t / mtiles) * 4 + wave, blocks = (V + 63) / 64;
     const int K4 = H / 4;
     // the block's piece k4 as a buffer load: the piece is a scalar offset (no vector address
-    // arithmetic beside the adds), and one past the block's end reads as zero
+    // arithmetic beside the adds), kept inside the block
     const auto e = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float4 *>(packed) + min(blk, blocks - 1) * K4 * 64, 0, K4 * 1024, 0x00020000);
     auto piece = [&](int at) {
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(e, lane * 16, at * 1024, 0));
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(e, lane * 16, nc::head_piece(at, K4) * 1024, 0));
     };
     f32x4 ring[kRing];
 #pragma unroll
