@@ -374,8 +374,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
 
 template <int T>
 int32_t launch_head_rows(void **p, const int64_t *s, int slots) {
-    const int64_t tiles = ((s[0] + T - 1) / T) * (((s[1] + 63) / 64 + 3) / 4);
-    hipLaunchKernelGGL((head_rows<T>), dim3((unsigned)tiles), dim3(256), 0, nc::stream(), (float *)p[0],
+    const unsigned workgroups = (unsigned)nc::head_workgroups(s[0], s[1], T);    // (head_tile: they fit)
+    hipLaunchKernelGGL((head_rows<T>), dim3(workgroups), dim3(256), 0, nc::stream(), (float *)p[0],
                        (unsigned long long *)p[1], (const float *)p[2], (const float4 *)p[3], (int)s[0], s[1],
                        (int)s[2], (const float *)p[5], (const float *)p[6], slots);
     return nc::launched("head_rows");
@@ -482,15 +482,11 @@ NC_EXPORT int32_t nc_lm_head(void **p, const int64_t *s) {
     const int64_t blocks = (s[1] + 63) / 64;
     const dim3 grid((unsigned)blocks, (unsigned)s[0]);
     const int slots = s[4] ? (int)grid.x : 0;
-    // Several rows: 16 a wave once that leaves two waves a SIMD, 4 a wave down to one wave a SIMD of
-    // the one-row kernels' (which read the table anew for every row, but whose
-    // many short waves hide what a few long ones cannot). Measured on MI355X, us, one row / 4 / 16 a wave:
-    // 128 x 151936 x 896: 10160 / 924 / 579; 16: 1272 / 167 / 124; 4: 322 / 104 / 122; 500 x 4864 x 896:
-    // 718 / 113 / 100; 128 x 4864 x 896: 141 / 39 / 50; 500 x 896 x 4864: 734 / 130 / 248;
-    // 16 x 4864 x 896: 21.1 / 20.3 / 49; 8 x 8192 x 8192: 228 / 195 / 410; 33 x 896 x 896: 10.6 / 20.6 / 49; 4 x 4864 x 896: 10.8 / 20.9 / 52.
-    if (s[0] > 1 && !p[4] && ((uintptr_t)p[2] & 15) == 0) {
-        if (s[0] > 4 && (s[0] + 15) / 16 * blocks >= 2048) return launch_head_rows<16>(p, s, slots);
-        if (s[0] * blocks >= 1000) return launch_head_rows<4>(p, s, slots);
+    // several rows (nc_rules.h says where the lines lie)
+    if (!p[4] && ((uintptr_t)p[2] & 15) == 0) {
+        const int tile = nc::head_tile(s[0], s[1]);
+        if (tile == 16) return launch_head_rows<16>(p, s, slots);
+        if (tile == 4) return launch_head_rows<4>(p, s, slots);
     }
     if (s[2] == 896) {       // the model's width: the ring kernel, 24 loads (24 KB) in flight per wave
         hipLaunchKernelGGL((lm_head_ring<896, 24>), grid, dim3(64), 0, nc::stream(), (float *)p[0],

@@ -11,4 +11,27 @@ namespace nc {
 // the index itself has to stay in the block, which may be the last of its allocation.
 constexpr int head_piece(int at, int pieces) { return at < pieces ? at : pieces - 1; }
 
+// HIP takes no launch of 2^32 or more threads along one dimension of the grid.
+constexpr bool grid_fits(int64_t workgroups, int64_t threads) { return workgroups < ((int64_t)1 << 32) / threads; }
+
+// Workgroups of the multi-row head (four waves, each one block of 64 table rows by `tile` rows of x),
+// along one dimension of its grid.
+constexpr int64_t head_workgroups(int64_t M, int64_t V, int tile) {
+    return (M + tile - 1) / tile * (((V + 63) / 64 + 3) / 4);
+}
+
+// Rows of x a wave of the LM head takes, for M rows by a table of V: 16 once that leaves two waves a SIMD,
+// 4 down to one wave a SIMD of the one-row kernels' (which read the table anew for every row, but whose
+// many short waves hide what a few long ones cannot), else 0: the one-row kernels, whose grid has the rows
+// along its second dimension, so they also take what the others' grid does not hold.
+// Measured on MI355X, us, one row / 4 / 16 a wave:
+// 128 x 151936 x 896: 10160 / 924 / 579; 16: 1272 / 167 / 124; 4: 322 / 104 / 122; 500 x 4864 x 896:
+// 718 / 113 / 100; 128 x 4864 x 896: 141 / 39 / 50; 500 x 896 x 4864: 734 / 130 / 248;
+// 16 x 4864 x 896: 21.1 / 20.3 / 49; 8 x 8192 x 8192: 228 / 195 / 410; 33 x 896 x 896: 10.6 / 20.6 / 49; 4 x 4864 x 896: 10.8 / 20.9 / 52.
+constexpr int head_tile(int64_t M, int64_t V) {
+    const int64_t blocks = (V + 63) / 64;
+    const int tile = M > 4 && (M + 15) / 16 * blocks >= 2048 ? 16 : M > 1 && M * blocks >= 1000 ? 4 : 0;
+    return tile && grid_fits(head_workgroups(M, V, tile), 256) ? tile : 0;
+}
+
 }  // namespace nc

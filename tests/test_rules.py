@@ -43,3 +43,13 @@ def test_a_head_prefetch_stays_in_its_block(run):
         }
     printf("%ld", bad);
     """) == "0"
+
+
+def test_head_tiles_fit_one_dimension_of_the_grid(run):
+    """Rows a wave of the multi-row head on both sides of its lines, and 0 (the one-row kernels) where its
+    workgroups of 256 threads would be 2^32 threads or more along the grid's first dimension."""
+    shapes = [(1, 151936, 0), (2, 32000, 4), (4, 151936, 4), (15, 4224, 0), (16, 4224, 4), (128, 151936, 16),
+              (65535, (1 << 20) - 256, 16), (65535, 1 << 20, 0), (65535, (1 << 28) + 256, 0),
+              (65535, (1 << 31) - 1, 0), (4, (1 << 31) - 1, 4)]
+    said = run("".join(f'printf("%d ", nc::head_tile({m}, {v}ll));' for m, v, _ in shapes)).split()
+    assert [int(t) for t in said] == [t for _, _, t in shapes]
