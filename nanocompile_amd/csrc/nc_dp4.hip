@@ -20,6 +20,7 @@
 // staging and two waves a SIMD.
 #include "nc_common.h"
 #include "nc_epilogue.h"
+#include "nc_rules.h"
 
 namespace {
 
@@ -219,8 +220,9 @@ __global__ __launch_bounds__(256) void matmul_i8_dp4(Dp4Args a) {
 
 template <int TM, int TN>
 int32_t launch_dp4(const Dp4Args &a) {
-    const unsigned tiles = (unsigned)((a.M + TM - 1) / TM * ((a.N + 8 * TN - 1) / (8 * TN)));
-    hipLaunchKernelGGL((matmul_i8_dp4<TM, TN>), dim3(tiles), dim3(256), 0, nc::stream(), a);
+    static_assert(TM == 8, "dp4_workgroups counts tiles of 8 rows");
+    const unsigned workgroups = (unsigned)nc::dp4_workgroups(a.M, a.N, TN);      // (dp4_columns: they fit)
+    hipLaunchKernelGGL((matmul_i8_dp4<TM, TN>), dim3(workgroups), dim3(256), 0, nc::stream(), a);
     return nc::launched("matmul_i8_dp4");
 }
 
@@ -228,23 +230,16 @@ int32_t launch_dp4(const Dp4Args &a) {
 
 namespace nc {
 
-// Few outputs stay with the kernels that give a chain a lane and every row of x its own workgroups
-// (nc_modes.hip): us, they / this kernel: 4 x 896 x 4864 6.4 / 11.8, 16 x 896 x 4864 11.3 / 11.9,
-// 1 x 8192 x 8192 21.3 / 23.8; 4 x 4864 x 896 6.4 / 6.1, 32 x 896 x 4864 19.0 / 12.1,
-// 128 x 896 x 4864 66.5 / 24.7, 128 x 4864 x 896 85.8 / 25.3, 100 x 8192 x 8192 900 / 187.
 bool matmul_i8_vnni_rows_ok(const int8_t *xq, const int8_t *packed, const int8_t *q, int64_t M, int64_t N) {
-    return M * N >= 16000 && (((uintptr_t)xq | (uintptr_t)packed | (uintptr_t)q) & 3) == 0;
+    return dp4_columns(M, N) && (((uintptr_t)xq | (uintptr_t)packed | (uintptr_t)q) & 3) == 0;
 }
 
-// 8 x 4 outputs a lane from 400 workgroups of them on, else 8 x 2 for twice the waves (32 x 896 x 4864
-// 12.1 against 17.6 us; 128 x 4864 x 896 26.7 against 25.3; 4 x 4 measured between the two).
 int32_t matmul_i8_vnni_rows(float *y, const int8_t *xq, const float *xs, const float *offset, const int8_t *packed,
                             const int8_t *q, const float *scales, const float *bias, const float *residual,
                             const float *gate, int64_t M, int64_t N, int64_t K, int64_t block) {
     const Dp4Args a{y,    xq,       xs,   offset, packed, q, scales,
                     bias, residual, gate, (int)M, (int)N, (int)K, __builtin_ctzll((unsigned long long)block)};
-    if ((M + 7) / 8 * ((N + 31) / 32) >= 400) return launch_dp4<8, 4>(a);
-    return launch_dp4<8, 2>(a);
+    return dp4_columns(M, N) == 4 ? launch_dp4<8, 4>(a) : launch_dp4<8, 2>(a);
 }
 
 }  // namespace nc

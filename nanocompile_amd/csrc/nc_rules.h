@@ -34,4 +34,24 @@ constexpr int head_tile(int64_t M, int64_t V) {
     return tile && grid_fits(head_workgroups(M, V, tile), 256) ? tile : 0;
 }
 
+// Workgroups of matmul_i8_vnni's register tiles (8 rows of x by 8 `columns` weight rows each), along one
+// dimension of its grid.
+constexpr int64_t dp4_workgroups(int64_t M, int64_t N, int columns) {
+    return (M + 7) / 8 * ((N + 8 * columns - 1) / (8 * columns));
+}
+
+// Weight rows a lane of matmul_i8_vnni's register tiles takes, or 0: the kernels that give a chain a lane
+// and every row of x its own workgroups along the grid's second dimension. Those keep the calls of few
+// outputs (us, they / the tiles: 4 x 896 x 4864 6.4 / 11.8, 16 x 896 x 4864 11.3 / 11.9,
+// 1 x 8192 x 8192 21.3 / 23.8; 4 x 4864 x 896 6.4 / 6.1, 32 x 896 x 4864 19.0 / 12.1,
+// 128 x 896 x 4864 66.5 / 24.7, 128 x 4864 x 896 85.8 / 25.3, 100 x 8192 x 8192 900 / 187), and those
+// whose tiles do not fit the grid. 4 from 400 workgroups of them on, else 2 for twice the waves
+// (32 x 896 x 4864 12.1 against 17.6 us; 128 x 4864 x 896 26.7 against 25.3; tiles of 4 rows by 4
+// measured between the two).
+constexpr int dp4_columns(int64_t M, int64_t N) {
+    if (M * N < 16000) return 0;
+    const int columns = dp4_workgroups(M, N, 4) >= 400 ? 4 : 2;
+    return grid_fits(dp4_workgroups(M, N, columns), 256) ? columns : 0;
+}
+
 }  // namespace nc

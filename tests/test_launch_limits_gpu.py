@@ -35,3 +35,30 @@ def test_argmax_keys_of_a_large_table(gpu):
             acc += x[row, k] * w[:, k]
         assert got[row] == acc.argmax(), row
     assert len(set(got.tolist())) > 1
+
+
+def rows_of(array, rows):
+    """Rows of a matrix on the device."""
+    n = array.shape[1]
+    return np.stack([array.view((n,), offset_bytes=4 * n * int(r)).numpy() for r in rows])
+
+
+def test_vnni_of_many_outputs(gpu, host):
+    """65,535 rows by 65,537 weight rows (2^32 outputs and more), the first and last rows bit for bit."""
+    from nanocompile_amd import hip
+    from nanocompile_amd.hip import DeviceArray
+    from oracle import reference as R
+    m, n, k = 65535, 65537, 32
+    print(f"matmul_i8_vnni m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(6)
+    rows = [0, 1, 7, 8, 40000, 65527, 65528, 65534]
+    xq = rng.integers(-127, 128, (m, k), dtype=np.int8)
+    xs, off = (rng.random((m, 1), dtype=np.float32) for _ in "so")
+    q, s = R.quantize_int8((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    y = DeviceArray((m, n), np.float32)
+    packed = DeviceArray.from_host(np.zeros(16, np.int8))        # no whole 128: the packed weights are not read
+    hip.call("nc_matmul_i8_vnni", [y, *map(DeviceArray.from_host, (xq, xs, off)), packed,
+                                   *map(DeviceArray.from_host, (q, s))], [m, n, k, 32])
+    hip.sync()
+    expected = host.matmul_i8_vnni(xq[rows], xs[rows], off[rows], q, s, 32)
+    assert np.array_equal(bits(rows_of(y, rows)), bits(expected))

@@ -53,3 +53,11 @@ def test_head_tiles_fit_one_dimension_of_the_grid(run):
               (65535, (1 << 31) - 1, 0), (4, (1 << 31) - 1, 4)]
     said = run("".join(f'printf("%d ", nc::head_tile({m}, {v}ll));' for m, v, _ in shapes)).split()
     assert [int(t) for t in said] == [t for _, _, t in shapes]
+
+
+def test_vnni_tiles_fit_one_dimension_of_the_grid(run):
+    """Weight rows a lane of matmul_i8_vnni's register tiles, 0 (a chain a lane) where they do not fit."""
+    shapes = [(4, 896, 0), (17, 896, 0), (18, 896, 2), (128, 4864, 4), (65535, 65504, 4), (65535, 65536, 0),
+              (65535, 65537, 0), (65535, (1 << 24) - 1, 0), (256, (1 << 24) - 32, 4), (257, (1 << 24) - 1, 0)]
+    said = run("".join(f'printf("%d ", nc::dp4_columns({m}, {n}ll));' for m, n, _ in shapes)).split()
+    assert [int(c) for c in said] == [c for _, _, c in shapes]
