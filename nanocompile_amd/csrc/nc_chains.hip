@@ -29,6 +29,7 @@
 // busy 76% of the time with 8-byte reads and four times the values traded through LDS.
 #include "nc_common.h"
 #include "nc_epilogue.h"
+#include "nc_rules.h"
 
 namespace {
 
@@ -240,8 +241,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 
 template <int MT, int NT, int NS>
 int32_t launch_chains(const ChainArgs &a) {
-    const unsigned tiles = (unsigned)((a.M + 16 * MT - 1) / (16 * MT) * ((a.N + 16 * NT - 1) / (16 * NT)));
-    hipLaunchKernelGGL((matmul_i8_chains<MT, NT, NS>), dim3(tiles), dim3(256), 0, nc::stream(), a);
+    static_assert(MT == 1, "chain_workgroups counts tiles of 16 rows");
+    const unsigned workgroups = (unsigned)nc::chain_workgroups(a.M, a.N, NT);    // (chain_tiles: they fit)
+    hipLaunchKernelGGL((matmul_i8_chains<MT, NT, NS>), dim3(workgroups), dim3(256), 0, nc::stream(), a);
     return nc::launched("matmul_i8_chains");
 }
 
@@ -249,24 +251,14 @@ int32_t launch_chains(const ChainArgs &a) {
 
 namespace nc {
 
-// At the model's widths the chain-a-lane kernel (nc_modes.hip) is as quick while the outputs are few: it
-// reads a weight row anew for every row of x but has 16 times the waves (us, it / this kernel: 16 x 896
-// x 4864 13.0 / 14.6, 24 x 896 x 4864 18.5 / 14.6, 4 x 4864 x 896 5.8 / 6.1, 6 x 4864 x 896 6.5 / 6.0,
-// 128 x 4864 x 896 88.5 / 16.4). Other widths' general kernel is slower throughout (1 x 8192 x 8192 65 /
-// 27, 100 x 8192 x 8192 6167 / 142, 1 x 1000 x 1000 5.8 / 5.7).
 bool matmul_i8_rows_ok(const float *x, const int8_t *packed, int64_t M, int64_t N, int64_t K) {
-    if (K < 32 || K % 8 != 0 || ((uintptr_t)x & 15) != 0 || ((uintptr_t)packed & 15) != 0) return false;
-    return M * N >= 20000 || (K != 896 && K != 4864);
+    return chain_tiles(M, N, K) && (((uintptr_t)x | (uintptr_t)packed) & 15) == 0;
 }
 
-// Two tiles of weight rows a workgroup once that leaves four workgroups a CU (128 x 4864 x 896: 16.4 us
-// against 18.0 with one; 128 x 896 x 4864, 224 such workgroups: 20.6 against 17.9). Tiles of 32 rows of x
-// measured no faster (32 x 32: 20.4, 512 x 4864 x 896 59.9 against 52.4).
 int32_t matmul_i8_rows(float *y, const float *x, const int8_t *packed, const int8_t *q, const float *scales,
                        const float *bias, const float *residual, const float *gate, int64_t M, int64_t N, int64_t K) {
     const ChainArgs a{y, x, packed, q, scales, bias, residual, gate, (int)M, (int)N, (int)K};
-    if ((M + 15) / 16 * ((N + 31) / 32) >= 1000) return launch_chains<1, 2, 2>(a);
-    return launch_chains<1, 1, 4>(a);
+    return chain_tiles(M, N, K) == 2 ? launch_chains<1, 2, 2>(a) : launch_chains<1, 1, 4>(a);
 }
 
 }  // namespace nc

@@ -11,7 +11,8 @@ namespace nc {
 // the index itself has to stay in the block, which may be the last of its allocation.
 constexpr int head_piece(int at, int pieces) { return at < pieces ? at : pieces - 1; }
 
-// HIP takes no launch of 2^32 or more threads along one dimension of the grid.
+// Whether a launch runs whole: a grid has fewer than 2^32 threads along one dimension. Past that the count
+// is cut to 32 bits (measured: the launch reports no error and most outputs are never written).
 constexpr bool grid_fits(int64_t workgroups, int64_t threads) { return workgroups < ((int64_t)1 << 32) / threads; }
 
 // Workgroups of the multi-row head (four waves, each one block of 64 table rows by `tile` rows of x),
@@ -52,6 +53,28 @@ constexpr int dp4_columns(int64_t M, int64_t N) {
     if (M * N < 16000) return 0;
     const int columns = dp4_workgroups(M, N, 4) >= 400 ? 4 : 2;
     return grid_fits(dp4_workgroups(M, N, columns), 256) ? columns : 0;
+}
+
+// Workgroups of matmul_i8 on the matrix cores (16 rows of x by 16 `tiles` weight rows each), along one
+// dimension of its grid.
+constexpr int64_t chain_workgroups(int64_t M, int64_t N, int tiles) {
+    return (M + 15) / 16 * ((N + 16 * tiles - 1) / (16 * tiles));
+}
+
+// Tiles of weight rows a workgroup of matmul_i8 on the matrix cores takes, or 0: the kernels that give
+// every row of x its own workgroups along the grid's second dimension. At the model's widths those run a
+// chain a lane and are as quick while the outputs are few: they read a weight row anew for every row of x
+// but have 16 times the waves (us, they / the matrix cores: 16 x 896 x 4864 13.0 / 14.6, 24 x 896 x 4864
+// 18.5 / 14.6, 4 x 4864 x 896 5.8 / 6.1, 6 x 4864 x 896 6.5 / 6.0, 128 x 4864 x 896 88.5 / 16.4). Other
+// widths' general kernel is slower throughout (1 x 8192 x 8192 65 / 27, 100 x 8192 x 8192 6167 / 142,
+// 1 x 1000 x 1000 5.8 / 5.7). Two tiles once that leaves four workgroups a CU (128 x 4864 x 896: 16.4 us
+// against 18.0 with one; 128 x 896 x 4864, 224 such workgroups: 20.6 against 17.9). Tiles of 32 rows of x
+// measured no faster (32 x 32: 20.4, 512 x 4864 x 896 59.9 against 52.4).
+constexpr int chain_tiles(int64_t M, int64_t N, int64_t K) {
+    if (K < 32 || K % 8 != 0) return 0;
+    if (M * N < 20000 && (K == 896 || K == 4864)) return 0;
+    const int tiles = chain_workgroups(M, N, 2) >= 1000 ? 2 : 1;
+    return grid_fits(chain_workgroups(M, N, tiles), 256) ? tiles : 0;
 }
 
 }  // namespace nc

@@ -1,4 +1,4 @@
-"""Calls whose workgroups do not fit one dimension of a grid (2^32 threads), a few rows of each against the oracle.
+"""Calls whose workgroups would not fit one dimension of a grid (2^32 threads), a few rows of each against the oracle.
 
 Long outputs over short dot products: gigabytes written in well under a second.
 """
@@ -62,3 +62,21 @@ def test_vnni_of_many_outputs(gpu, host):
     hip.sync()
     expected = host.matmul_i8_vnni(xq[rows], xs[rows], off[rows], q, s, 32)
     assert np.array_equal(bits(rows_of(y, rows)), bits(expected))
+
+
+def test_int8_of_many_outputs(gpu, host):
+    """65,535 rows by 131,073 weight rows (2^33 outputs and more), the first and last rows bit for bit."""
+    from nanocompile_amd import hip
+    from nanocompile_amd.hip import DeviceArray
+    from nanocompile_amd.kernels import pack_chains
+    from oracle import reference as R
+    m, n, k = 65535, 131073, 32
+    print(f"matmul_i8 m={m} n={n} k={k}", flush=True)
+    rng = np.random.default_rng(7)
+    rows = [0, 1, 15, 16, 40000, 65519, 65520, 65534]
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    q, s = R.quantize_int8((rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    y = DeviceArray((m, n), np.float32)
+    hip.call("nc_matmul_i8", [y, *map(DeviceArray.from_host, (x, pack_chains(q), q, s))], [m, n, k])
+    hip.sync()
+    assert np.array_equal(bits(rows_of(y, rows)), bits(host.matmul_i8_f32(x[rows], q, s)))

@@ -61,3 +61,12 @@ def test_vnni_tiles_fit_one_dimension_of_the_grid(run):
               (65535, 65537, 0), (65535, (1 << 24) - 1, 0), (256, (1 << 24) - 32, 4), (257, (1 << 24) - 1, 0)]
     said = run("".join(f'printf("%d ", nc::dp4_columns({m}, {n}ll));' for m, n, _ in shapes)).split()
     assert [int(c) for c in said] == [c for _, _, c in shapes]
+
+
+def test_int8_tiles_fit_one_dimension_of_the_grid(run):
+    """Tiles a workgroup of matmul_i8 on the matrix cores, 0 (the kernels of a grid row a row) where they do not fit."""
+    shapes = [(16, 896, 4864, 0), (24, 896, 4864, 1), (128, 4864, 896, 2), (128, 896, 4864, 1), (20, 70, 24, 0),
+              (20, 70, 100, 0), (65535, 131040, 32, 2), (65535, 131072, 32, 0), (65535, (1 << 24) - 1, 32, 0),
+              (512, (1 << 24) - 33, 40, 2), (512, (1 << 24) - 1, 40, 0)]
+    said = run("".join(f'printf("%d ", nc::chain_tiles({m}, {n}ll, {k}));' for m, n, k, _ in shapes)).split()
+    assert [int(t) for t in said] == [t for *_, t in shapes]
