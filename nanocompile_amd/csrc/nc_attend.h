@@ -243,18 +243,20 @@ __device__ __forceinline__ void chunk_scores_sq(const float *__restrict__ q, flo
 }
 
 // (keys from n on have p = 0 and leave the accumulators unchanged, so the key
-// loop stops at the first group of four that holds none of the n keys)
+// loop stops at the first group of four that holds none of the n keys; in the
+// group that holds the last of them, the values from n on are taken as zeros: a
+// prompt's later rows are staged too, and 0 times an infinite one is not 0)
 template <int D, int H>
 __device__ __forceinline__ void chunk_values_n(float (*qp)[kChunk], const Staged<D> &st, int n, float (&o)[H]) {
     const int lane = threadIdx.x & 63;
     const int dl = lane < D ? lane : 0;
 #pragma unroll
     for (int u = 0; u < H; ++u) o[u] = 0.0f;
-    const int groups = (n + 3) >> 2;
-#pragma unroll 2
-    for (int i = 0; i < groups; ++i) {
-        const float v0 = st.values[(4 * i + 0) * D + dl], v1 = st.values[(4 * i + 1) * D + dl];
-        const float v2 = st.values[(4 * i + 2) * D + dl], v3 = st.values[(4 * i + 3) * D + dl];
+    auto step = [&](int i, int seen) {
+        const float v0 = st.values[(4 * i + 0) * D + dl];
+        const float v1 = seen > 1 ? st.values[(4 * i + 1) * D + dl] : 0.0f;
+        const float v2 = seen > 2 ? st.values[(4 * i + 2) * D + dl] : 0.0f;
+        const float v3 = seen > 3 ? st.values[(4 * i + 3) * D + dl] : 0.0f;
 #pragma unroll
         for (int u = 0; u < H; ++u) {
             const float4 pi = *reinterpret_cast<const float4 *>(qp[u] + 4 * i);
@@ -263,7 +265,11 @@ __device__ __forceinline__ void chunk_values_n(float (*qp)[kChunk], const Staged
             o[u] = __builtin_fmaf(pi.z, v2, o[u]);
             o[u] = __builtin_fmaf(pi.w, v3, o[u]);
         }
-    }
+    };
+    const int whole = n >> 2;
+#pragma unroll 2
+    for (int i = 0; i < whole; ++i) step(i, 4);
+    if (n & 3) step(whole, n & 3);
 }
 
 // Store a chunk result at part[0 .. D + 1] (m_j, l_j, o_j).

@@ -18,12 +18,12 @@ from tests.conftest import bits
 pytestmark = pytest.mark.gpu
 
 
-def attend(host, heads, kv, d, m, past, spoil=None, slab=None):
+def attend(host, heads, kv, d, m, past, spoil=None, slab=None, schedule=0):
     """(ctx, xq, xs) of the GPU and of the oracle for one seeded prompt."""
     from nanocompile_amd import hip
     from nanocompile_amd.hip import DeviceArray
     from nanocompile_amd.kernels import attention_workspace_bytes, float_bits
-    print(f"attention heads={heads}/{kv} d={d} m={m} past={past} slab={slab}", flush=True)
+    print(f"attention heads={heads}/{kv} d={d} m={m} past={past} slab={slab} schedule={schedule}", flush=True)
     rng = np.random.default_rng(heads + 3 * m + 7 * past)
     cap = past + m + 3
     qkv = rng.standard_normal((m, (heads + 2 * kv) * d)).astype(np.float32)
@@ -38,7 +38,7 @@ def attend(host, heads, kv, d, m, past, spoil=None, slab=None):
     work, ctx = DeviceArray((nbytes // 4,), np.float32), DeviceArray((m, heads * d), np.float32)
     xq, xs = DeviceArray((m, heads * d), np.int8), DeviceArray((m,), np.float32)
     hip.call("nc_attention", [ctx, dq, dk, dv, None, work, xq, xs],
-             [m, heads, kv, d, past, cap, float_bits(scale), nbytes])
+             [m, heads, kv, d, past, cap, float_bits(scale), nbytes, schedule])
     hip.sync()
     return ctx.numpy(), xq.numpy(), xs.numpy(), expected
 
@@ -64,6 +64,25 @@ def test_values_a_row_must_not_see(gpu, host, m, past):
     ctx, _, _, expected = attend(host, heads, kv, d, m, past, spoil)
     assert np.isfinite(ctx[:at]).all()
     assert np.array_equal(bits(ctx[:at]), bits(expected[:at]))
+    assert np.array_equal(np.isnan(ctx), np.isnan(expected))
+    assert np.array_equal(ctx[~np.isnan(ctx)], expected[~np.isnan(ctx)])
+
+
+@pytest.mark.parametrize("heads,kv,d,schedule", [*((14, 2, 64, s) for s in (1, 2, 3, 4)), (8, 8, 64, 0), (66, 1, 16, 0)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_values_no_schedule_may_see(gpu, host, heads, kv, d, schedule, bad):
+    """Every schedule, and groups the matrix cores do not take: an infinite or NaN value of each later key of
+    a chunk (every remainder of a row's keys by four) reaches no earlier row."""
+    m, past = 26, 50
+    spoiled = {16: 2, 19: 0, 21: 3, 22: 1}                      # row: element (keys 66, 69, 71, 72)
+
+    def spoil(qkv, kc, vc):
+        for row, e in spoiled.items():
+            qkv[row, (heads + kv) * d + e] = bad                # a value of KV head 0
+    ctx, xq, xs, expected = attend(host, heads, kv, d, m, past, spoil, schedule=schedule)
+    first = min(spoiled)
+    assert np.isfinite(ctx[:first]).all()
+    assert np.array_equal(bits(ctx[:first]), bits(expected[:first]))
     assert np.array_equal(np.isnan(ctx), np.isnan(expected))
     assert np.array_equal(ctx[~np.isnan(ctx)], expected[~np.isnan(ctx)])
 
