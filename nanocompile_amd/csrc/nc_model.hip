@@ -484,7 +484,7 @@ NC_EXPORT int32_t nc_lm_head(void **p, const int64_t *s) {
     const int slots = s[4] ? (int)grid.x : 0;
     // several rows (nc_rules.h says where the lines lie)
     if (!p[4] && ((uintptr_t)p[2] & 15) == 0) {
-        const int tile = nc::head_tile(s[0], s[1]);
+        const int tile = nc::head_tile(s[0], s[1], s[2]);
         if (tile == 16) return launch_head_rows<16>(p, s, slots);
         if (tile == 4) return launch_head_rows<4>(p, s, slots);
     }

@@ -21,17 +21,49 @@ constexpr int64_t head_workgroups(int64_t M, int64_t V, int tile) {
     return (M + tile - 1) / tile * (((V + 63) / 64 + 3) / 4);
 }
 
-// Rows of x a wave of the LM head takes, for M rows by a table of V: 16 once that leaves two waves a SIMD,
-// 4 down to one wave a SIMD of the one-row kernels' (which read the table anew for every row, but whose
-// many short waves hide what a few long ones cannot), else 0: the one-row kernels, whose grid has the rows
-// along its second dimension, so they also take what the others' grid does not hold.
-// Measured on MI355X, us, one row / 4 / 16 a wave:
-// 128 x 151936 x 896: 10160 / 924 / 579; 16: 1272 / 167 / 124; 4: 322 / 104 / 122; 500 x 4864 x 896:
-// 718 / 113 / 100; 128 x 4864 x 896: 141 / 39 / 50; 500 x 896 x 4864: 734 / 130 / 248;
-// 16 x 4864 x 896: 21.1 / 20.3 / 49; 8 x 8192 x 8192: 228 / 195 / 410; 33 x 896 x 896: 10.6 / 20.6 / 49; 4 x 4864 x 896: 10.8 / 20.9 / 52.
-constexpr int head_tile(int64_t M, int64_t V) {
+// The part of a packed table of V rows by H that one XCD reads when every row of x reads it anew, in bytes.
+// Workgroup i of a launch runs on XCD i mod 8, so 64-row block b of the table goes to XCD (b + m blocks) mod 8
+// for row m of x: always to the same one where the blocks are a multiple of 8, to all 8 where they are odd.
+constexpr int64_t head_slice(int64_t V, int64_t H) {
     const int64_t blocks = (V + 63) / 64;
-    const int tile = M > 4 && (M + 15) / 16 * blocks >= 2048 ? 16 : M > 1 && M * blocks >= 1000 ? 4 : 0;
+    const int64_t parts = blocks % 8 == 0 ? 8 : blocks % 4 == 0 ? 4 : blocks % 2 == 0 ? 2 : 1;
+    return blocks * 64 * H * 4 / parts;
+}
+
+// Rows of x a wave of the LM head takes, for M rows of H by a table of V rows: 16, 4, or 0 (the one-row
+// kernels, whose grid has the rows along its second dimension, so they also take what the others' grid
+// does not hold).
+//
+// 16 once that leaves two waves a SIMD. Measured on MI355X, us, one row / 4 / 16 a wave: 128 x 151936 x 896:
+// 10160 / 924 / 579; 16: 1272 / 167 / 124; 4: 322 / 104 / 122; 500 x 4864 x 896: 718 / 113 / 100;
+// 128 x 4864 x 896: 141 / 39 / 50; 500 x 896 x 4864: 734 / 130 / 248; 8 x 8192 x 8192: 228 / 195 / 410.
+//
+// 4 against the one-row kernels: with up to about 4,000 (row, block) pairs its waves are one to a SIMD and it
+// takes the time of one wave's k loop whatever their number (H = 64 / 128 / 256 / 512 / 896 / 2048 / 4096:
+// 5.2 / 6.2 / 8.7 / 13.7 / 21.3 / 44 / 95 us), where the one-row kernels' time grows with the pairs, each of
+// which reads 256 H bytes, and with the memory those come from: an XCD's L2 (4 MB) while its slice of the
+// table stays there, slower memory past that. Pairs at which the two are equal: a slice under 1.8 MB
+// 2,100-2,700 (2800 x 64 x 896 of 2,304 rows 25.6 / 21.4), 2 MB 1,400-1,800, more than 2.3 MB under 1,000,
+// except at the model's width, whose ring kernel is better there (6400 rows: 1,000 pairs 18.8 / 21.3, 1,200
+// 23.9 / 21.3) until the slice passes every L2; rows of 128 and less about 2,700; rows of 4,096 about 1,150
+// (512 x 4096: 1,000 pairs 78 / 94, 1,400 108 / 94), of 8,192 under 1,000. A table of one block leaves three of
+// a workgroup's four waves without work: four times the pairs (4000 x 64 x 896 33.7 / 45.0, 8000 77.4 / 83.8).
+constexpr int64_t head_pairs(int64_t V, int64_t H) {
+    const int64_t slice = head_slice(V, H);
+    int64_t pairs = 2300;
+    if (H >= 8192) pairs = 1000;
+    else if (slice >= 2300000) pairs = H == 896 && slice < 20000000 ? 1100 : 1000;
+    else if (H >= 4096) pairs = 1150;
+    else if (H <= 128) pairs = 2700;
+    else if (slice >= 1800000 && H != 896) pairs = 1600;
+    return V <= 64 && H < 4096 ? 4 * pairs : pairs;
+}
+
+constexpr int head_tile(int64_t M, int64_t V, int64_t H) {
+    const int64_t blocks = (V + 63) / 64;
+    const int tile = M > 4 && (M + 15) / 16 * blocks >= 2048 ? 16
+                     : M > 1 && M * blocks >= head_pairs(V, H) ? 4
+                                                               : 0;
     return tile && grid_fits(head_workgroups(M, V, tile), 256) ? tile : 0;
 }
 

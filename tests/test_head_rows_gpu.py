@@ -30,6 +30,9 @@ def in_order(x, w):
     (17, 65537, 60),           # 16 rows a wave: a remainder of one, no whole stage, one row past a block
     (16, 131071, 132),         # the last block short, rows not a multiple of 4 (no 16-byte stores)
     (333, 6400, 128),
+    (2, 90000, 68),            # 4 rows a wave of a narrow table: two rows of four, one piece past a stage
+    (7, 25500, 132),           # rows of the table not a whole block, x one row short of two fours
+    (10805, 1, 64),            # one table row, three of four waves without work
 ])
 @pytest.mark.parametrize("epilogue", [False, True])
 def test_rows_match_the_reference_order(gpu, m, v, h, epilogue):

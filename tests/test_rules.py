@@ -46,13 +46,26 @@ def test_a_head_prefetch_stays_in_its_block(run):
 
 
 def test_head_tiles_fit_one_dimension_of_the_grid(run):
-    """Rows a wave of the multi-row head on both sides of its lines, and 0 (the one-row kernels) where its
-    workgroups of 256 threads would be 2^32 threads or more along the grid's first dimension."""
-    shapes = [(1, 151936, 0), (2, 32000, 4), (4, 151936, 4), (15, 4224, 0), (16, 4224, 4), (128, 151936, 16),
-              (65535, (1 << 20) - 256, 16), (65535, 1 << 20, 0), (65535, (1 << 28) + 256, 0),
-              (65535, (1 << 31) - 1, 0), (4, (1 << 31) - 1, 4)]
-    said = run("".join(f'printf("%d ", nc::head_tile({m}, {v}ll));' for m, v, _ in shapes)).split()
-    assert [int(t) for t in said] == [t for _, _, t in shapes]
+    """Rows a wave of the multi-row head, and 0 (the one-row kernels) where its workgroups of 256 threads
+    would be 2^32 threads or more along the grid's first dimension."""
+    shapes = [(1, 151936, 896, 0), (2, 151936, 896, 4), (4, 151936, 896, 4), (128, 151936, 896, 16),
+              (65535, (1 << 20) - 256, 4, 16), (65535, 1 << 20, 4, 0), (65535, (1 << 28) + 256, 4, 0),
+              (65535, (1 << 31) - 1, 4, 0), (4, (1 << 31) - 1, 4, 4)]
+    said = run("".join(f'printf("%d ", nc::head_tile({m}, {v}ll, {h}));' for m, v, h, _ in shapes)).split()
+    assert [int(t) for t in said] == [t for *_, t in shapes]
+
+
+def test_head_rows_where_they_are_quicker(run):
+    """The one-row kernels where they measured quicker than four rows a wave, four rows where those did."""
+    one_row = [(64, 1024, 1024), (500, 128, 1024), (100, 896, 896), (56, 1152, 896), (2, 32768, 128), (500, 128, 128),
+               (1000, 64, 64), (4000, 64, 896), (175, 512, 256), (32, 2048, 512), (8, 8192, 896), (10, 6400, 896),
+               (42, 3072, 896), (125, 1024, 2048), (125, 512, 4096), (71, 1536, 1536)]
+    four = [(2, 32000, 896), (3, 24000, 4096), (8, 8192, 1024), (128, 512, 8192), (400, 896, 896), (17, 8192, 896),
+            (72, 896, 4864), (350, 512, 512), (88, 2048, 896), (16, 4864, 896), (32, 8192, 64), (10, 6400, 512),
+            (22, 3000, 1536), (175, 512, 4096), (1000, 512, 64), (2000, 64, 4096)]
+    said = run("".join(f'printf("%d ", nc::head_tile({m}, {v}, {h}));' for m, v, h in one_row + four)).split()
+    wrong = [(s, t) for s, t in zip(one_row + four, said) if int(t) != (0 if s in one_row else 4)]
+    assert not wrong
 
 
 def test_vnni_tiles_fit_one_dimension_of_the_grid(run):
