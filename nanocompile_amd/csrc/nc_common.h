@@ -201,7 +201,8 @@ bool matmul_i8_rows_ok(const float *x, const int8_t *packed, int64_t M, int64_t 
 int32_t matmul_i8_rows(float *y, const float *x, const int8_t *packed, const int8_t *q, const float *scales,
                        const float *bias, const float *residual, const float *gate, int64_t M, int64_t N, int64_t K);
 // matmul_i8_vnni over several rows in register tiles (nc_dp4.hip), and whether it takes a problem.
-bool matmul_i8_vnni_rows_ok(const int8_t *xq, const int8_t *packed, const int8_t *q, int64_t M, int64_t N);
+bool matmul_i8_vnni_rows_ok(const int8_t *xq, const int8_t *packed, const int8_t *q, int64_t M, int64_t N,
+                            int64_t K);
 int32_t matmul_i8_vnni_rows(float *y, const int8_t *xq, const float *xs, const float *offset, const int8_t *packed,
                             const int8_t *q, const float *scales, const float *bias, const float *residual,
                             const float *gate, int64_t M, int64_t N, int64_t K, int64_t block);

@@ -230,8 +230,8 @@ int32_t launch_dp4(const Dp4Args &a) {
 
 namespace nc {
 
-bool matmul_i8_vnni_rows_ok(const int8_t *xq, const int8_t *packed, const int8_t *q, int64_t M, int64_t N) {
-    return dp4_columns(M, N) && (((uintptr_t)xq | (uintptr_t)packed | (uintptr_t)q) & 3) == 0;
+bool matmul_i8_vnni_rows_ok(const int8_t *xq, const int8_t *packed, const int8_t *q, int64_t M, int64_t N, int64_t K) {
+    return dp4_columns(M, N, K) && (((uintptr_t)xq | (uintptr_t)packed | (uintptr_t)q) & 3) == 0;
 }
 
 int32_t matmul_i8_vnni_rows(float *y, const int8_t *xq, const float *xs, const float *offset, const int8_t *packed,
@@ -239,7 +239,7 @@ int32_t matmul_i8_vnni_rows(float *y, const int8_t *xq, const float *xs, const f
                             const float *gate, int64_t M, int64_t N, int64_t K, int64_t block) {
     const Dp4Args a{y,    xq,       xs,   offset, packed, q, scales,
                     bias, residual, gate, (int)M, (int)N, (int)K, __builtin_ctzll((unsigned long long)block)};
-    return dp4_columns(M, N) == 4 ? launch_dp4<8, 4>(a) : launch_dp4<8, 2>(a);
+    return dp4_columns(M, N, K) == 4 ? launch_dp4<8, 4>(a) : launch_dp4<8, 2>(a);
 }
 
 }  // namespace nc

@@ -776,7 +776,7 @@ NC_EXPORT int32_t nc_matmul_i8_vnni(void **p, const int64_t *s) {
                    (block & (block - 1)) == 0 && K % block == 0,
                "nc_matmul_i8_vnni: bad shape (block a power of two >= 32 dividing K)");
     if (M == 0 || N == 0) return NC_OK;
-    if (nc::matmul_i8_vnni_rows_ok((const int8_t *)p[1], (const int8_t *)p[4], (const int8_t *)p[5], M, N))
+    if (nc::matmul_i8_vnni_rows_ok((const int8_t *)p[1], (const int8_t *)p[4], (const int8_t *)p[5], M, N, K))
         return nc::matmul_i8_vnni_rows((float *)p[0], (const int8_t *)p[1], (const float *)p[2], (const float *)p[3],
                                        (const int8_t *)p[4], (const int8_t *)p[5], (const float *)p[6],
                                        (const float *)p[7], (const float *)p[8], nullptr, M, N, K, block);
@@ -808,7 +808,7 @@ NC_EXPORT int32_t nc_matmul_i8_vnni_silu(void **p, const int64_t *s) {
                    (block & (block - 1)) == 0 && K % block == 0 && ((uintptr_t)p[1] & 15) == 0,
                "nc_matmul_i8_vnni_silu: bad shape (K 896 or 4864, block a power of two >= 32 dividing K)");
     if (M == 0 || N == 0) return NC_OK;
-    if (nc::matmul_i8_vnni_rows_ok((const int8_t *)p[1], (const int8_t *)p[4], (const int8_t *)p[5], M, N))
+    if (nc::matmul_i8_vnni_rows_ok((const int8_t *)p[1], (const int8_t *)p[4], (const int8_t *)p[5], M, N, K))
         return nc::matmul_i8_vnni_rows((float *)p[0], (const int8_t *)p[1], (const float *)p[2], (const float *)p[3],
                                        (const int8_t *)p[4], (const int8_t *)p[5], (const float *)p[6], nullptr, nullptr,
                                        (const float *)p[7], M, N, K, block);

@@ -74,15 +74,24 @@ constexpr int64_t dp4_workgroups(int64_t M, int64_t N, int columns) {
 }
 
 // Weight rows a lane of matmul_i8_vnni's register tiles takes, or 0: the kernels that give a chain a lane
-// and every row of x its own workgroups along the grid's second dimension. Those keep the calls of few
-// outputs (us, they / the tiles: 4 x 896 x 4864 6.4 / 11.8, 16 x 896 x 4864 11.3 / 11.9,
-// 1 x 8192 x 8192 21.3 / 23.8; 4 x 4864 x 896 6.4 / 6.1, 32 x 896 x 4864 19.0 / 12.1,
-// 128 x 896 x 4864 66.5 / 24.7, 128 x 4864 x 896 85.8 / 25.3, 100 x 8192 x 8192 900 / 187), and those
-// whose tiles do not fit the grid. 4 from 400 workgroups of them on, else 2 for twice the waves
-// (32 x 896 x 4864 12.1 against 17.6 us; 128 x 4864 x 896 26.7 against 25.3; tiles of 4 rows by 4
-// measured between the two).
-constexpr int dp4_columns(int64_t M, int64_t N) {
+// and every row of x its own workgroups along the grid's second dimension. Those keep (us, they / the tiles):
+// * the calls of few outputs: 4 x 896 x 4864 6.4 / 11.8, 16 x 896 x 4864 11.3 / 11.9; 4 x 4864 x 896 6.4 / 6.1,
+//   32 x 896 x 4864 19.0 / 12.1, 128 x 896 x 4864 66.5 / 24.7, 128 x 4864 x 896 85.8 / 25.3,
+//   100 x 8192 x 8192 900 / 187;
+// * one row (a tile's other seven are copies of it; with the quantizer's launch 1 x 16000 x 896 10.7 / 12.1,
+//   1 x 65536 x 2048 30.7 / 42.3, 1 x 151936 x 896 32.4 / 48.9), but for long rows by few weight rows at widths
+//   other than the model's, where the general kernel has too few waves (1 x 16000 x 4096 28.7 / 26.9,
+//   1 x 16000 x 8192 52.4 / 46.0, 1 x 32768 x 16384 203 / 162; 1 x 24000 x 4096 32.3 / 34.4,
+//   1 x 32768 x 8192 72.5 / 78.0);
+// * two rows of less than 512 (2 x 65536 x 256 13.9 / 17.3; 2 x 16000 x 512 10.8 / 10.1; three rows
+//   3 x 65536 x 256 17.3 / 17.3);
+// * what does not fit the tiles' grid.
+// 4 from 400 workgroups of them on, else 2 for twice the waves (32 x 896 x 4864 12.1 against 17.6 us;
+// 128 x 4864 x 896 26.7 against 25.3; tiles of 4 rows by 4 measured between the two).
+constexpr int dp4_columns(int64_t M, int64_t N, int64_t K) {
     if (M * N < 16000) return 0;
+    if (M == 1 && (K == 896 || K == 4864 || N > 4 * K || (N >= 32768 && N > 2 * K))) return 0;
+    if (M == 2 && K < 512) return 0;
     const int columns = dp4_workgroups(M, N, 4) >= 400 ? 4 : 2;
     return grid_fits(dp4_workgroups(M, N, columns), 256) ? columns : 0;
 }

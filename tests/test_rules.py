@@ -70,10 +70,21 @@ def test_head_rows_where_they_are_quicker(run):
 
 def test_vnni_tiles_fit_one_dimension_of_the_grid(run):
     """Weight rows a lane of matmul_i8_vnni's register tiles, 0 (a chain a lane) where they do not fit."""
-    shapes = [(4, 896, 0), (17, 896, 0), (18, 896, 2), (128, 4864, 4), (65535, 65504, 4), (65535, 65536, 0),
-              (65535, 65537, 0), (65535, (1 << 24) - 1, 0), (256, (1 << 24) - 32, 4), (257, (1 << 24) - 1, 0)]
-    said = run("".join(f'printf("%d ", nc::dp4_columns({m}, {n}ll));' for m, n, _ in shapes)).split()
-    assert [int(c) for c in said] == [c for _, _, c in shapes]
+    shapes = [(4, 896, 4864, 0), (17, 896, 896, 0), (18, 896, 896, 2), (128, 4864, 896, 4), (65535, 65504, 32, 4),
+              (65535, 65536, 32, 0), (65535, 65537, 32, 0), (65535, (1 << 24) - 1, 32, 0),
+              (256, (1 << 24) - 32, 32, 4), (257, (1 << 24) - 1, 32, 0)]
+    said = run("".join(f'printf("%d ", nc::dp4_columns({m}, {n}ll, {k}));' for m, n, k, _ in shapes)).split()
+    assert [int(c) for c in said] == [c for *_, c in shapes]
+
+
+def test_vnni_tiles_where_they_are_quicker(run):
+    """A chain a lane where that measured quicker than the register tiles, the tiles where they did."""
+    chains = [(1, 16000, 896), (1, 32000, 896), (1, 151936, 64), (1, 65536, 2048), (1, 151936, 4864), (1, 24000, 4096),
+              (1, 16000, 4864), (1, 32768, 8192), (1, 151936, 8192), (2, 65536, 256), (2, 16000, 128)]
+    tiles = [(1, 16384, 4096), (1, 16000, 8192), (1, 32768, 16384), (2, 16000, 512), (2, 8192, 8192), (2, 151936, 896),
+             (3, 16000, 256), (3, 65536, 896), (4, 4864, 896), (500, 64, 128)]
+    said = run("".join(f'printf("%d ", nc::dp4_columns({m}, {n}, {k}));' for m, n, k in chains + tiles)).split()
+    assert [s for s, c in zip(chains + tiles, said) if (int(c) > 0) != (s in tiles)] == []
 
 
 def test_int8_tiles_fit_one_dimension_of_the_grid(run):
