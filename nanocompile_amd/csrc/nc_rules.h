@@ -102,18 +102,37 @@ constexpr int64_t chain_workgroups(int64_t M, int64_t N, int tiles) {
     return (M + 15) / 16 * ((N + 16 * tiles - 1) / (16 * tiles));
 }
 
-// Tiles of weight rows a workgroup of matmul_i8 on the matrix cores takes, or 0: the kernels that give
-// every row of x its own workgroups along the grid's second dimension. At the model's widths those run a
-// chain a lane and are as quick while the outputs are few: they read a weight row anew for every row of x
-// but have 16 times the waves (us, they / the matrix cores: 16 x 896 x 4864 13.0 / 14.6, 24 x 896 x 4864
-// 18.5 / 14.6, 4 x 4864 x 896 5.8 / 6.1, 6 x 4864 x 896 6.5 / 6.0, 128 x 4864 x 896 88.5 / 16.4). Other
-// widths' general kernel is slower throughout (1 x 8192 x 8192 65 / 27, 100 x 8192 x 8192 6167 / 142,
-// 1 x 1000 x 1000 5.8 / 5.7). Two tiles once that leaves four workgroups a CU (128 x 4864 x 896: 16.4 us
-// against 18.0 with one; 128 x 896 x 4864, 224 such workgroups: 20.6 against 17.9). Tiles of 32 rows of x
-// measured no faster (32 x 32: 20.4, 512 x 4864 x 896 59.9 against 52.4).
+// Whether matmul_i8 of M rows by N weight rows is quicker on the matrix cores, whose tiles of 16 rows of x
+// read a weight row once, than on the kernels that give every row of x its own workgroups: a chain a lane at
+// the model's widths, four chains a lane at any other (us, they / the matrix cores).
+// Model's widths: few outputs stay with a chain a lane, which has 16 times the waves (16 x 896 x 4864
+// 13.0 / 14.6, 24 x 896 x 4864 18.5 / 14.6, 6 x 4864 x 896 6.5 / 6.0, 128 x 4864 x 896 88.5 / 16.4), and so do
+// few rows, of which a tile is mostly copies: one row always (20000 x 896 6.0 / 11.2, 65536 x 4864 79 / 107), two
+// (40000 x 896 16.7 / 17.7, 25000 x 4864 44.8 / 46.4, 65536 x 896 26.3 / 25.4), three or four of 896
+// (3 x 6667 5.9 / 6.9, 4 x 5000 5.9 / 6.9, 4 x 7500 8.0 / 6.9).
+// Other widths, from four rows on: 512 and wider always (4 x 4096 x 512 5.4 / 5.1, 256 x 256 x 512 7.4 / 5.3),
+// below that from some outputs on (8 x 2048 x 256 4.6 / 4.8, 8 x 4096 x 256 5.1 / 4.8).
+// One to three rows: 3072 and wider always (1 x 8192 x 3072 22.1 / 13.2); 1536 to 3071 but for one row by many
+// (1 x 8192 x 1536 9.0 / 8.7, 1 x 24000 x 1536 15.4 / 18.2, 1 x 24000 x 2048 20.3 / 22.5); 512 to 1535 by few
+// weight rows (1 x 4096 x 1024 6.8 / 6.2, 2 x 8192 x 1000 7.3 / 7.9, 1 x 16384 x 1024 7.2 / 9.9), or by enough
+// of them for the second and third row to pay (3 x 10923 x 768 9.3 / 7.6, 2 x 65536 x 1024 31.3 / 28.3); narrower
+// never (1 x 65536 x 64 5.2 / 8.6).
+constexpr bool chains_pay(int64_t M, int64_t N, int64_t K) {
+    if (K == 896 || K == 4864)
+        return M > 1 && M * N >= (M == 2 ? 100000 : M <= 4 && K == 896 ? 28000 : 20000);
+    if (M >= 4) return K >= 512 || M * N >= (K >= 384 ? 16000 : 24000);
+    if (K >= 3072) return true;
+    if (K >= 1536) return M > 1 || N <= (K >= 2048 ? 20000 : 8192);
+    if (K < 512) return false;
+    return N <= 4096 || (M == 3 && K >= 768) || (M == 2 && K >= 1000 && N >= 40000);
+}
+
+// Tiles of weight rows a workgroup of matmul_i8 on the matrix cores takes, or 0: the kernels of a grid row a row
+// of x. Two once that leaves four workgroups a CU (128 x 4864 x 896: 16.4 us against 18.0 with one;
+// 128 x 896 x 4864, 224 such workgroups: 20.6 against 17.9). Tiles of 32 rows of x measured no faster
+// (32 x 32: 20.4, 512 x 4864 x 896 59.9 against 52.4).
 constexpr int chain_tiles(int64_t M, int64_t N, int64_t K) {
-    if (K < 32 || K % 8 != 0) return 0;
-    if (M * N < 20000 && (K == 896 || K == 4864)) return 0;
+    if (K < 32 || K % 8 != 0 || !chains_pay(M, N, K)) return 0;
     const int tiles = chain_workgroups(M, N, 2) >= 1000 ? 2 : 1;
     return grid_fits(chain_workgroups(M, N, tiles), 256) ? tiles : 0;
 }

@@ -26,7 +26,10 @@ def operands(m, n, k):
 
 
 SHAPES = [(1, 17, 32), (17, 33, 40), (5, 100, 104), (16, 16, 128), (33, 31, 136), (18, 50, 216), (1, 70, 1000),
-          (40, 500, 160), (256, 2001, 96), (23, 896, 896), (24, 896, 4864), (130, 3900, 896)]
+          (40, 500, 160), (256, 2001, 96), (23, 896, 896), (24, 896, 4864), (130, 3900, 896),
+          # the matrix cores' least outputs and widths, every remainder of a width by 128 and by 32
+          (257, 97, 32), (33, 731, 40), (5, 4803, 104), (6, 4001, 128), (17, 1433, 136), (18, 1351, 216), (40, 601, 160),
+          (16, 16, 640), (4, 17, 520), (7, 33, 552), (19, 50, 744), (1, 31, 3096), (2, 20, 1560), (3, 5, 512)]
 
 
 @pytest.mark.parametrize("m,n,k", SHAPES)

@@ -94,3 +94,15 @@ def test_int8_tiles_fit_one_dimension_of_the_grid(run):
               (512, (1 << 24) - 33, 40, 2), (512, (1 << 24) - 1, 40, 0)]
     said = run("".join(f'printf("%d ", nc::chain_tiles({m}, {n}ll, {k}));' for m, n, k, _ in shapes)).split()
     assert [int(t) for t in said] == [t for *_, t in shapes]
+
+
+def test_int8_on_the_matrix_cores_where_it_is_quicker(run):
+    """The kernels of a grid row a row of x where they measured quicker, the matrix cores where those did."""
+    rows = [(1, 20000, 896), (1, 151936, 896), (2, 10000, 896), (3, 6667, 896), (4, 5000, 896), (1, 65536, 4864),
+            (2, 13000, 4864), (1, 65536, 64), (2, 151936, 128), (64, 64, 256), (16, 1024, 128), (1, 16384, 512),
+            (2, 8192, 1000), (1, 32768, 1024), (1, 48000, 1536), (1, 65536, 2048)]
+    cores = [(3, 20000, 896), (4, 7500, 896), (22, 1000, 896), (3, 7000, 4864), (2, 65536, 4864), (8, 65536, 896),
+             (512, 64, 128), (4, 16384, 512), (256, 256, 96), (8, 4096, 256), (1, 4096, 1024), (3, 10923, 1000),
+             (2, 65536, 1024), (1, 8192, 2048), (1, 16384, 4096), (1, 65536, 8192), (2, 16384, 1536)]
+    said = run("".join(f'printf("%d ", nc::chain_tiles({m}, {n}, {k}));' for m, n, k in rows + cores)).split()
+    assert [s for s, t in zip(rows + cores, said) if (int(t) > 0) != (s in cores)] == []
