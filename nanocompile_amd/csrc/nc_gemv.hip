@@ -19,6 +19,7 @@
 // the group applies the epilogue.
 #include "nc_common.h"
 #include "nc_epilogue.h"
+#include "nc_rules.h"
 
 namespace {
 
@@ -269,20 +270,6 @@ int auto_tile(int M, int N, int K) {
     return 2;
 }
 
-// The SwiGLU pair's default: 64 x 64 with two register stages (its tiles
-// stage two weight blocks, so deeper rings cost occupancy) from 400 such
-// tiles, else 32 x 32 (measured at N = 4864, K = 896: M = 384 / 512 / 1024 /
-// 2048: 15.7 / 19.3 / 30.5 / 54.1 us against 16.8 / 20.6 / 35.2 / 68.1 with
-// 32 x 32 and 17.3 / 20.6 / 34.9 / 63.3 with 32 x 64; M = 128 / 256: 8.41 /
-// 12.13 us with 32 x 32 against 11.0 / 14.6 with 64 x 64). Long k loops (K >= 2048) take 64 x 64 from
-// 200 tiles (100 x 8000 x 4096: 19.4 against 22.8 with 32 x 32) and 128 x 64 past 256 (350 x 4000 x 2560:
-// 16.6 against 19.8 and 22.4).
-int auto_tile_pair(int M, int N, int K) {
-    const int t64 = ((M + 63) / 64) * ((N + 63) / 64);
-    if (K >= 2048 && t64 > 256) return 8;
-    return t64 >= (K >= 2048 ? 200 : 400) ? 5 : 2;
-}
-
 template <int KS, int MT, bool ACC_OUT>
 int32_t dispatch_schedule(const Args &a, int schedule) {
 #define NC_GEMV_CASE(I, L, W) \
@@ -431,7 +418,7 @@ NC_EXPORT int32_t nc_matmul_i8_token_swiglu(void **p, const int64_t *s) {
     auto sg = (const float *)p[4];
     auto qu = (const int8_t *)p[5];
     auto su = (const float *)p[6];
-    if (schedule == 0 && M >= kGemmMinTokens) schedule = kGemmFirst + auto_tile_pair(M, N, K);
+    if (schedule == 0 && M >= kGemmMinTokens) schedule = kGemmFirst + nc::pair_tile(M, N, K);
     if (schedule >= kGemmFirst)
         return nc::gemm_i8_token(schedule - kGemmFirst, 2, h, xq, xs, qg, sg, nullptr, nullptr, qu, su, M, N, K);
     if (K == 896) return swiglu_tokens<896>(h, xq, xs, qg, sg, qu, su, M, N, K);

@@ -137,4 +137,26 @@ constexpr int chain_tiles(int64_t M, int64_t N, int64_t K) {
     return grid_fits(chain_workgroups(M, N, tiles), 256) ? tiles : 0;
 }
 
+// The SwiGLU pair's MFMA tile (nc_gemm.hip): 2 is 32 x 32, 5 is 64 x 64 with two register stages (its tiles
+// stage two weight blocks, so deeper rings cost occupancy), 8 is 128 x 64.
+// Short k loops: 64 x 64 from 400 such tiles, else 32 x 32 (measured at N = 4864, K = 896: M = 384 / 512 / 1024 /
+// 2048: 15.7 / 19.3 / 30.5 / 54.1 us against 16.8 / 20.6 / 35.2 / 68.1 with 32 x 32 and 17.3 / 20.6 / 34.9 / 63.3
+// with 32 x 64; M = 128 / 256: 8.41 / 12.13 us with 32 x 32 against 11.0 / 14.6 with 64 x 64).
+// Long k loops (K >= 2048; us, 32 x 32 / 64 x 64 / 128 x 64): 128 x 64 past 256 tiles of 64 x 64 while its own
+// fit one a CU (190 x 8000 x 4096 34.4 / 28.4 / 25.7, 512 x 3000 x 2048 19.9 / 18.0 / 15.7), or fill whole rounds
+// of that without more padding (500 x 8192 x 2048 47.5 / 33.0 / 31.0); a round begun costs it what a full one does
+// (257 x 6400 x 2048, 300 of them, 24.3 / 19.2 / 25.4; 1000 x 4864 x 2048, 608, 55.0 / 39.0 / 42.9), and up to 64
+// rows half of each is padding (32 x 16500 x 2048 16.5 / 18.4 / 25.5). Else 64 x 64 from 400 tiles, or from 200
+// to 256 where it pads little more than 32 x 32 (64 x 13000 x 2048 16.5 / 14.9 / 16.7; 200 x 3300 x 2048
+// 11.7 / 12.8 / 14.8).
+constexpr int pair_tile(int64_t M, int64_t N, int64_t K) {
+    const int64_t n64 = (N + 63) / 64, t64 = (M + 63) / 64 * n64, t128 = (M + 127) / 128 * n64;
+    const int64_t t32 = (M + 31) / 32 * ((N + 31) / 32);
+    if (K < 2048) return t64 >= 400 ? 5 : 2;
+    const int64_t rounds = (t128 + 255) / 256;
+    const bool whole = 100 * t128 >= 98 * 256 * rounds && 20 * t128 <= 11 * t64;
+    if (t64 > 256 && (t128 <= 256 || whole)) return 8;
+    return t64 >= 400 || (t64 >= 200 && t64 <= 256 && 40 * t64 <= 11 * t32) ? 5 : 2;
+}
+
 }  // namespace nc

@@ -106,3 +106,16 @@ def test_int8_on_the_matrix_cores_where_it_is_quicker(run):
              (2, 65536, 1024), (1, 8192, 2048), (1, 16384, 4096), (1, 65536, 8192), (2, 16384, 1536)]
     said = run("".join(f'printf("%d ", nc::chain_tiles({m}, {n}, {k}));' for m, n, k in rows + cores)).split()
     assert [s for s, t in zip(rows + cores, said) if (int(t) > 0) != (s in cores)] == []
+
+
+def test_pair_tiles_where_they_are_quicker(run):
+    """The SwiGLU pair's tile at shapes of long k loops where each of 32 x 32, 64 x 64 and 128 x 64 measured quickest."""
+    quickest = {2: [(32, 16500, 2048), (16, 20000, 2048), (64, 16500, 2048), (60, 20000, 2048), (64, 20000, 4096),
+                    (200, 3300, 2048), (128, 4864, 896)],
+                5: [(64, 13000, 2048), (100, 8000, 2048), (64, 26000, 2048), (257, 6400, 2048), (700, 3000, 3072),
+                    (400, 4864, 2560), (300, 8192, 4096), (130, 16384, 2048), (1000, 4864, 2048), (512, 4864, 896)],
+                8: [(190, 8000, 4096), (130, 8192, 4096), (100, 12800, 2048), (512, 3000, 2048), (260, 4096, 4096),
+                    (384, 4096, 4096), (500, 8192, 2048), (2000, 2000, 4096)]}
+    shapes = [(t, s) for t in quickest for s in quickest[t]]
+    said = run("".join(f'printf("%d ", nc::pair_tile({m}, {n}, {k}));' for _, (m, n, k) in shapes)).split()
+    assert [(s, int(got)) for (t, s), got in zip(shapes, said) if int(got) != t] == []
