@@ -26,6 +26,7 @@
 #include "nc_epilogue.h"
 #include "nc_exp.h"
 #include "nc_math.h"
+#include "nc_rules.h"
 
 namespace {
 
@@ -156,8 +157,8 @@ __global__ __launch_bounds__(kThreads) void rope_append(float *__restrict__ qkv,
 // e = 0 (m_j), 1 (l_j), 2 + d (o_j[d]); jstride = the chunks of the longest
 // context of the call.
 constexpr int kWaves = 8;              // decode: waves of a chunk workgroup, one query head each
-// Prefill on the vector ALU (attention_rows_chunks: the schedules 1 .. 4, and groups of more
-// than 64 heads): 4 query rows per workgroup, one per wave. A wave attends its row's
+// Prefill on the vector ALU (attention_rows_chunks: the schedules 1 .. 4, small groups over little
+// work, and groups of more than 64 heads): 4 query rows per workgroup, one per wave. A wave attends its row's
 // heads of the group together, up to 7 at a time (nc_attend.h's
 // chunk_scores_sq and chunk_values_n: every key or value element read from LDS
 // once for all the heads' chains, the row's queries read with scalar loads
@@ -172,9 +173,8 @@ constexpr int kWaves = 8;              // decode: waves of a chunk workgroup, on
 // of that one-head kernel, all slower: 8, 2 or 1 rows a workgroup (62, 63, 99
 // us), registers capped at three waves a SIMD (spills: 168 us), each head's
 // query read with scalar loads (69-73 us).
-constexpr int kRowsPerBlock = 4;         // prefill: query rows (waves) a chunk workgroup, the library's choice
 // The prefill schedules a tuner may choose: schedule s (1..4) stages each
-// chunk for kScheduleRows[s - 1] rows; schedule 0 is attention_rows_mfma. Every
+// chunk for kScheduleRows[s - 1] rows; schedule 0 is the library's choice (prefill_rows). Every
 // choice computes the same bits: a row's arithmetic does not depend on which
 // workgroup holds it.
 constexpr int kScheduleRows[4] = {2, 4, 8, 16};
@@ -914,8 +914,7 @@ NC_EXPORT int32_t nc_attention(void **p, const int64_t *s) {
     if (M == 0) return NC_OK;
     const float scale = nc::bits_to_float(s[6]);
     float *work = (float *)p[5];
-    // schedule 0: the matrix cores while a KV head's group of query heads fits a workgroup's 64 columns
-    const int rows = schedule ? kScheduleRows[schedule - 1] : heads / kv <= 64 ? 0 : kRowsPerBlock;
+    const int rows = schedule ? kScheduleRows[schedule - 1] : nc::prefill_rows(M, heads, kv, pos ? cap : past + M);
 #define NC_PREFILL(R)                                                                             \
     if (rows == R) {                                                                              \
         if (D == 64) return launch_prefill<64, R>(p, M, heads, kv, past, cap, scale, pos, work, work_bytes); \

@@ -159,4 +159,20 @@ constexpr int pair_tile(int64_t M, int64_t N, int64_t K) {
     return t64 >= 400 || (t64 >= 200 && t64 <= 256 && 40 * t64 <= 11 * t32) ? 5 : 2;
 }
 
+// Query rows a workgroup of a prompt's chunk kernel takes by the library's choice, for M rows and at most `keys`
+// keys: 0 is attention_rows_mfma, 4 is attention_rows_chunks<D, 4>. The matrix cores take 64 (row, head) pairs
+// of a KV head's group at a time, so they need the group to fit that, and a small group needs many rows to fill
+// it: with up to four heads a group and little work the vector ALU's smaller workgroups are quicker, in
+// proportion to (blocks of 4 rows) x chunks x heads (us, vector ALU / matrix cores, with the combine: 8 heads of 8,
+// 64 rows at past 0 8.8 / 11.1, past 400 (1,024) 10.8 / 11.6, past 1200 (2,560) 21.3 / 13.2; 4 of 4 by 32,
+// 128 rows at past 400 (1,152) 10.4 / 10.9, 64 at 1200 (1,280) 11.5 / 11.3; 16 of 8, 64 rows at past 100 (768)
+// 10.9 / 12.0, 128 rows (2,048) 12.6 / 12.5; 12 of 4, 128 rows at past 0 (768) 10.6 / 11.6, 256 (3,072)
+// 13.5 / 12.4; 8 of 2 by 32, 64 rows at past 400 (1,024) 10.3 / 11.1, 128 (2,304) 12.3 / 11.6). Groups of 6 and
+// more are quicker on the matrix cores at every size (14 of 2, 2 rows at past 0 10.3 / 9.2).
+constexpr int prefill_rows(int64_t M, int64_t heads, int64_t kv_heads, int64_t keys) {
+    const int64_t group = heads / kv_heads;
+    if (group > 64) return 4;
+    return group <= 4 && (M + 3) / 4 * ((keys + 63) / 64) * heads <= 1200 ? 4 : 0;
+}
+
 }  // namespace nc

@@ -45,7 +45,9 @@ def attend(host, heads, kv, d, m, past, spoil=None, slab=None, schedule=0):
 
 @pytest.mark.parametrize("heads,kv,d,m,past", [
     (3, 3, 64, 130, 0), (14, 2, 64, 10, 57), (14, 2, 64, 19, 500), (33, 1, 64, 5, 61), (64, 1, 32, 3, 130),
-    (66, 1, 16, 4, 60), (17, 17, 16, 70, 64), (6, 2, 64, 9, 4090), (4, 2, 32, 600, 7)])
+    (66, 1, 16, 4, 60), (17, 17, 16, 70, 64), (6, 2, 64, 9, 4090), (4, 2, 32, 600, 7),
+    # small groups with enough rows for the matrix cores
+    (3, 3, 64, 300, 200), (17, 17, 16, 70, 300), (6, 2, 64, 40, 4050), (2, 2, 32, 521, 100), (8, 2, 16, 130, 400)])
 @pytest.mark.parametrize("slab", [None, 4])
 def test_prompt_attention(gpu, host, heads, kv, d, m, past, slab):
     ctx, xq, xs, expected = attend(host, heads, kv, d, m, past, slab=slab)
