@@ -439,10 +439,12 @@ class Qwen2:
     def _fused_norm(self, k: int, m: int) -> bool:
         """Whether int8 mode's qkv projection takes the first norm in (nc_matmul_i8_normed, the
         model's widths; the residual stream is 256-byte aligned in the arena). Only there: its
-        144 workgroups repeat the norm's chain in one round, where the gate and up projections'
-        608 each would repeat it over several (measured slower); and only for a few tokens, as
-        from 16 on the projection without the norm runs on the matrix cores (the same bits)."""
-        return self.quantization == "int8" and k in (896, 4864) and m < 16
+        144 workgroups a token repeat the norm's chain in one round, where the gate and up
+        projections' 608 each would repeat it over several (measured slower); and only up to 14
+        tokens, whose workgroups (at most 2,016) are all resident at once: the norm in a launch of
+        its own gives the same bits and is quicker from there on (us, taken in / of its own:
+        8 tokens 7.8 / 9.2, 14 8.6 / 10.1, 15 13.1 / 10.7, 17 13.7 / 11.0, 64 32.4 / 12.1)."""
+        return self.quantization == "int8" and k in (896, 4864) and m < 15
 
     def _silu_epilogue(self, k: int) -> bool:
         """Whether the reference modes' up projection applies SwiGLU in its epilogue
