@@ -196,7 +196,7 @@ def call(name: str, pointers, sizes) -> None:
     try:
         p = _POINTERS[len(pointers)].pack(*[x if x.__class__ is int else _address(x) or 0 for x in pointers])
         s = _SIZES[len(sizes)].pack(*sizes)
-    except (struct.error, IndexError):     # more than PAD entries, or sizes that are not whole numbers of 64 bits
+    except (struct.error, IndexError, TypeError):   # more than PAD entries, or sizes not whole numbers of 64 bits
         p = bytes((ctypes.c_void_p * max(PAD, len(pointers)))(*[_address(x) for x in pointers]))
         s = bytes((ctypes.c_int64 * max(PAD, len(sizes)))(*[int(v) for v in sizes]))
     status = fn(p, s)

@@ -17,7 +17,8 @@ class Array:
 
 @pytest.mark.parametrize("pointers,sizes", [
     ([], []), ([None, 5, Array(1 << 47)], [1, np.int64(2), True, -3]), ((7,), (1.9, np.float32(2.0))),
-    (list(range(1, 17)), list(range(16))), (list(range(1, 21)), list(range(-4, 14))), ([0, -8], [2 ** 63, -2 ** 63])])
+    (list(range(1, 17)), list(range(16))), (list(range(1, 21)), list(range(-4, 14))), ([0, -8], [2 ** 63, -2 ** 63]),
+    ([], [np.array(2.0), np.array(3), np.float64(4.0)])])
 def test_arguments(monkeypatch, pointers, sizes):
     seen = []
     # a c_char_p argument is the bytes object itself, not its text up to the first zero
