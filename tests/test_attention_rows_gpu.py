@@ -18,7 +18,7 @@ from tests.conftest import bits
 pytestmark = pytest.mark.gpu
 
 
-def attend(host, heads, kv, d, m, past, spoil=None, slab=None, schedule=0):
+def attend(host, heads, kv, d, m, past, spoil=None, slab=None, schedule=0, scale=None):
     """(ctx, xq, xs) of the GPU and of the oracle for one seeded prompt."""
     from nanocompile_amd import hip
     from nanocompile_amd.hip import DeviceArray
@@ -30,7 +30,7 @@ def attend(host, heads, kv, d, m, past, spoil=None, slab=None, schedule=0):
     kc, vc = (rng.standard_normal((kv, cap, d)).astype(np.float32) for _ in "kv")
     if spoil:
         spoil(qkv, kc, vc)
-    inv, scale = inverse_frequencies(d, 1e6), float(np.float32(d ** -0.5))
+    inv, scale = inverse_frequencies(d, 1e6), float(np.float32(d ** -0.5 if scale is None else scale))
     dq, dk, dv, dinv = (DeviceArray.from_host(a) for a in (qkv, kc, vc, inv))
     expected = host.rope_append_attention(qkv, kc, vc, inv, heads, kv, d, past, scale)
     hip.call("nc_rope_append", [dq, dk, dv, dinv], [m, heads, kv, d, past, cap])

@@ -117,3 +117,27 @@ def test_block_quantizer_rows(gpu, k, aligned):
     assert np.array_equal(bits(xs.numpy()[finite]), bits(es[finite]))
     assert np.array_equal(bits(off.numpy()[finite]), bits(eoff[finite, 0]))
     assert np.array_equal(np.isnan(xs.numpy()), np.isnan(es)) and np.array_equal(np.isinf(xs.numpy()), np.isinf(es))
+
+
+@pytest.mark.parametrize("k", [32, 96, 1024, 1056])
+def test_block_quantizer_rows_agree(gpu, k):
+    """The two routes' bytes, scales and offsets over NaN and infinite elements at every place of a block."""
+    from nanocompile_amd import hip
+    from nanocompile_amd.hip import DeviceArray
+    m = 128
+    rng = np.random.default_rng(k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    for i, bad in enumerate([np.nan, np.inf, -np.inf, -0.0]):
+        x[32 * i + np.arange(32), np.arange(32) + 32 * (i % (k // 32))] = bad
+    room = DeviceArray((m * k + 1,), np.float32)
+    got = []
+    for at in (0, 4):
+        room.upload(np.concatenate([x.reshape(-1), [0]] if at == 0 else [[0], x.reshape(-1)]).astype(np.float32))
+        outs = DeviceArray((m, k), np.int8), DeviceArray((m, k // 32), np.float32), DeviceArray((m,), np.float32)
+        hip.call("nc_quantize_blocks", [*outs, room.ptr + at], [m, k, 32])
+        hip.sync()
+        got.append([o.numpy() for o in outs])
+    assert np.array_equal(got[0][0], got[1][0])
+    for a, b in zip(got[0][1:], got[1][1:]):
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(bits(a)[~np.isnan(a)], bits(b)[~np.isnan(b)])
+    assert np.isnan(got[0][1]).any() and np.isinf(got[0][1]).any()
