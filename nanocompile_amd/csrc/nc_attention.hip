@@ -842,7 +842,8 @@ int32_t launch_prefill(void **p, int64_t M, int64_t heads, int64_t kv, int64_t p
     const int64_t host_past = pos ? 0 : past;
     for (int64_t i0 = 0; i0 < M; i0 += slab) {
         const int64_t rows = std::min(slab, M - i0);
-        if (ROWS == 0) {
+        int32_t rc;
+        if constexpr (ROWS == 0) {
             const int64_t R = 64 / (heads / kv), blocks = (rows + R - 1) / R;
             auto chunks_of = [&](int64_t z) { return (past + i0 + std::min((z + 1) * R, rows) - 1) / nc::kChunk + 1; };
             int64_t most = blocks > 1 ? 2 * jstride : jstride;   // chunks of a z of the grid: one block's, or two's
@@ -855,16 +856,16 @@ int32_t launch_prefill(void **p, int64_t M, int64_t heads, int64_t kv, int64_t p
                                dim3(256), 0, nc::stream(), work, (const float *)p[1], (const float *)p[2],
                                (const float *)p[3], (int)heads, (int)kv, (int)host_past, (int)cap, scale, (int)i0,
                                (int)rows, (int)M, (int)jstride, (int)R, pos, nc::error_word());
+            rc = nc::launched("attention_rows_mfma");
         } else {
-            constexpr int WAVES = ROWS ? ROWS : 1;
             const int64_t chunks = pos ? jstride : (past + i0 + rows + nc::kChunk - 1) / nc::kChunk;
-            hipLaunchKernelGGL((attention_rows_chunks<D, WAVES>),
-                               dim3((unsigned)chunks, (unsigned)kv, (unsigned)((rows + WAVES - 1) / WAVES)),
-                               dim3(64 * WAVES), 0, nc::stream(), work, (const float *)p[1], (const float *)p[2],
+            hipLaunchKernelGGL((attention_rows_chunks<D, ROWS>),
+                               dim3((unsigned)chunks, (unsigned)kv, (unsigned)((rows + ROWS - 1) / ROWS)),
+                               dim3(64 * ROWS), 0, nc::stream(), work, (const float *)p[1], (const float *)p[2],
                                (const float *)p[3], (int)heads, (int)kv, (int)host_past, (int)cap, scale, (int)i0,
                                (int)rows, (int)M, (int)jstride, pos, nc::error_word());
+            rc = nc::launched("attention_rows_chunks");
         }
-        int32_t rc = nc::launched("attention_rows_chunks");
         if (rc == NC_OK)
             rc = whole_rows ? launch_combine_rows<D>(p, fused, work, heads, host_past, cap, i0, rows, M, jstride, pos)
                             : launch_combine<D>((float *)p[0], work, heads, host_past, cap, i0, rows, M, jstride, pos);
