@@ -332,18 +332,21 @@ int32_t nc_matmul_i8_token_rope(void **p, const int64_t *s);
  * reference's repeat_kv as index arithmetic, nn.py:109-120). The softmax and
  * the context are computed in 64-key chunks combined afterwards, the order
  * nc_attention_decode shares, so prefill and decode agree bit for bit. One
- * workgroup per (64-key chunk, KV head, 4 query rows) attends the rows' query
- * heads of the group to its chunk; a second launch combines the chunks. The
- * reference materializes the [heads, M, keys] scores instead (README.md:317).
+ * workgroup per (64-key chunk, KV head, block of query rows) attends the rows'
+ * query heads of the group to its chunk, on the float32 matrix cores (up to 64
+ * (row, head) pairs at a time) or, for small groups over little work and groups
+ * of more than 64 heads, 4 rows on the vector ALU; a second launch combines the
+ * chunks. The reference materializes the [heads, M, keys] scores instead (README.md:317).
  * With xq and xs, ctx's per-token int8 (nc_quantize_token_i8's bits) is written
- * too, by the combine itself when a row's chunk results fit its LDS.
+ * too, by the combine itself for rows of at most 16 heads and 64 chunks.
  * p: [ctx f32[M,heads*D], qkv (q rotated), kcache, vcache, pos i64[1] or NULL,
  *     work f32 (the chunk results: heads * ceil(keys / 64) * (D + 2) floats per query
  *     row, keys = C with pos, else past + M; fewer than M rows' worth takes the rows
  *     in slabs), xq i8[M,heads*D] or NULL, xs f32[M] or NULL];
  * s: [M, heads, kv, D, past, C, scale as float32 bits, work bytes, schedule] (D 16, 32 or 64;
- *    at most 16384 keys; schedule 0 the library's query rows a chunk workgroup, 1..4 the
- *    tuner's choices, nc_attention_schedule_info; every schedule the same bits) */
+ *    at most 16384 keys; schedule 0 the library's choice, 1..4 the tuner's: 2, 4, 8
+ *    or 16 query rows a workgroup on the vector ALU, nc_attention_schedule_info; every
+ *    schedule the same bits) */
 int32_t nc_attention(void **p, const int64_t *s);
 
 /* A prefill attention schedule, for the tuner (no device call): out = [query rows a chunk

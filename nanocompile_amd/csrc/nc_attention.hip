@@ -176,7 +176,9 @@ constexpr int kWaves = 8;              // decode: waves of a chunk workgroup, on
 // The prefill schedules a tuner may choose: schedule s (1..4) stages each
 // chunk for kScheduleRows[s - 1] rows; schedule 0 is the library's choice (prefill_rows). Every
 // choice computes the same bits: a row's arithmetic does not depend on which
-// workgroup holds it.
+// workgroup holds it. Against schedule 0 they gain where a few rows of a small group meet a long
+// context (8 rows of 8 heads of 8 at past 4,000: 13.7 us with 8 rows a workgroup, 15.5 with 4, 16.9 on the
+// matrix cores; 16 heads of 8 17.9, 19.4 and 20.1); over 318 other shapes the best of them is at most 7% ahead.
 constexpr int kScheduleRows[4] = {2, 4, 8, 16};
 constexpr int kHeadBatch = 7;          // prefill: query heads of a row held in LDS at once (a group, in Qwen2)
 
@@ -282,13 +284,15 @@ __global__ __launch_bounds__(64 * ROWS) void attention_rows_chunks(
 // infinite or NaN: a chunk holding such a value that some row of the block must not
 // see is taken a row at a time, the masked values as zeros.
 //
-// The float32 matrix instructions and the vector ALU share their units (a loop of both
-// took the sum of their times), so the bound is 128 multiply-adds a (query, key) at the
-// 77 T/s the instructions reach alone plus the softmax's vector instructions, about as
-// much again: 2,048 rows, 50 + 45 us; measured with the combine 164 us, against 242 with
-// attention_rows_chunks (512 rows: 21.7 against 25.8). What is left there is the chunk
-// results (125 MB written and read) and the short life of a workgroup; 32 queries a wave,
-// for half the LDS reads, measured slower (177 and 25.1: fewer, longer workgroups).
+// The float32 matrix instructions and the vector ALU share their units (a loop of both took the
+// sum of their times: 32 cycles a matrix instruction and 2.2 a vector one, several waves on a SIMD),
+// so the bound is 128 multiply-adds a (query, key) at the 77 T/s the instructions reach alone plus the
+// softmax's vector instructions: 2,048 rows, 3.8 M matrix instructions (50 us) and 20.6 M others (18 us at
+// that rate; the exponentials' double steps are slower). Measured with the combine 168 us, against 242 with
+// attention_rows_chunks (512 rows: 21.7 against 25.8); the matrix instructions alone keep the units busy
+// half of the time a CU has work. What is left is the chunk results (125 MB written and read) and the short
+// life of a workgroup; 32 queries a wave, for half the LDS reads, measured slower (177 and 25.1: fewer, longer
+// workgroups).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef f32x4 __attribute__((aligned(8))) f32x4_at8;      // a chunk result is D + 2 floats: 8-byte aligned
@@ -509,7 +513,7 @@ __global__ __launch_bounds__(64) void attention_combine(float *__restrict__ ctx,
 }
 
 // The combine of one query over a long context: grid (heads, rows), four waves that bring
-// the chunk results to LDS together (16 loads a thread in flight, 62 chunks at D = 64),
+// the chunk results to LDS together (8 loads of two floats a thread in flight, 62 chunks at D = 64),
 // then one wave in combine_chunks' order.
 template <int D>
 __global__ __launch_bounds__(256) void attention_combine_wide(float *__restrict__ ctx, const float *__restrict__ part,
@@ -897,8 +901,7 @@ int32_t launch_decode(void **p, const int64_t *s, const int64_t *pos, float *wor
 // p: [ctx f32[M, heads*D], qkv f32[M, (H + 2*KV*D)] (q rotated), kcache, vcache, pos i64[1] | NULL,
 //     work f32[...], xq i8[M, heads*D] | NULL, xs f32[M] | NULL (with both: ctx's per-token int8 too)];
 // s: [M, heads, kv_heads, D, past, capacity, scale as float32 bits, work bytes, schedule]
-//    (D 16, 32 or 64; schedule 0 the library's rows a workgroup, 1..4 the tuner's choices:
-//    nc_attention_schedule_info)
+//    (D 16, 32 or 64; schedule 0 the library's choice, 1..4 the tuner's: nc_attention_schedule_info)
 // With pos, past is read from the device when the kernels run (s[4] is ignored). The workspace
 // holds the chunk results; one query row needs heads * ceil(keys / 64) * (D + 2) floats, keys =
 // past + M (capacity with pos), and a smaller workspace than M rows' takes the rows in slabs.

@@ -194,13 +194,15 @@ __global__ __launch_bounds__(64) void lm_head_ring(float *logits, unsigned long 
 // one k with a zero accumulator is the rounded product (a * b + 0; a product of
 // -0 becomes +0, and no partial sum is ever -0, so adding either leaves the
 // same bits), for 64 table rows and T rows of x at once. What is left for the
-// vector ALU is the one add a product needs, which bounds it: 128 rows of the
-// model's head are 17.4 G adds, 443 us at 64 lanes a cycle a CU; measured 579 us,
-// where a launch of one-row waves, each reading the table anew, took 10,160.
+// vector ALU is the one add a product needs. The two share their units (a loop of
+// both takes the sum of their times: an add 2.2 cycles with several waves on a
+// SIMD, a product instruction 32), which bounds it: 128 rows of the model's head
+// are 17.4 G products, 222 us of them and 244 of adds; measured 567 us, where a
+// launch of one-row waves, each reading the table anew, takes 10,280.
 // (32 rows a wave, a 32 x 32 instruction: 611; without the products issued a step
 // ahead: 592, and 355 against 248 us where a wave runs alone on its SIMD.)
 //
-// One wave owns a 64-row block of the table and MG times T rows of x. The packed
+// One wave owns a 64-row block of the table and T rows of x. The packed
 // layout is the instruction's first operand as it stands (lane l: row l, four
 // consecutive k a 16-byte load), so table values go from memory to registers,
 // kRing 1-KB loads ahead; x goes through LDS, 64 k a stage, shared by the
@@ -210,7 +212,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // The products of one k: `of` gives the lane kQuads quads, quad q holding
-// table rows row(q, lane) .. + 3 of the block for row x_row(lane) of x.
+// table rows row(q, lane) .. + 3 of the block for row lane % T of x.
 template <int T>
 struct Products;
 
