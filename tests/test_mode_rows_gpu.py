@@ -53,11 +53,11 @@ def test_matmul_i8_rows(gpu, host, m, n, k):
         assert np.array_equal(bits(h.numpy()), bits(want.numpy()))
 
 
-def test_matmul_i8_rows_unaligned_operands(gpu, host):
+@pytest.mark.parametrize("m,n,k", [(20, 70, 160), (20, 1300, 160), (30, 900, 896)])
+def test_matmul_i8_rows_unaligned_operands(gpu, host, m, n, k):
     """x 4 bytes past a 16-byte boundary takes the kernel that reads it an element at a time."""
     from nanocompile_amd import hip, kernels
     from nanocompile_amd.hip import DeviceArray
-    m, n, k = 20, 70, 160
     _, x, q, s = operands(m, n, k)
     room = DeviceArray((m * k + 1,), np.float32)
     room.upload(np.concatenate([[0], x.reshape(-1)]).astype(np.float32))
