@@ -168,7 +168,8 @@ constexpr int pair_tile(int64_t M, int64_t N, int64_t K) {
 // 128 rows at past 400 (1,152) 10.4 / 10.9, 64 at 1200 (1,280) 11.5 / 11.3; 16 of 8, 64 rows at past 100 (768)
 // 10.9 / 12.0, 128 rows (2,048) 12.6 / 12.5; 12 of 4, 128 rows at past 0 (768) 10.6 / 11.6, 256 (3,072)
 // 13.5 / 12.4; 8 of 2 by 32, 64 rows at past 400 (1,024) 10.3 / 11.1, 128 (2,304) 12.3 / 11.6). Groups of 6 and
-// more are quicker on the matrix cores at every size (14 of 2, 2 rows at past 0 10.3 / 9.2).
+// more are quicker on the matrix cores at every size (14 of 2, 2 rows at past 0 10.3 / 9.2), of 5 as quick
+// (10 of 2, 64 rows at past 0 10.9 / 11.1, at past 400 12.3 / 12.0).
 constexpr int prefill_rows(int64_t M, int64_t heads, int64_t kv_heads, int64_t keys) {
     const int64_t group = heads / kv_heads;
     if (group > 64) return 4;

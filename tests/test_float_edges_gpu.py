@@ -25,8 +25,8 @@ def head(x, w):
     from nanocompile_amd import hip
     from nanocompile_amd.hip import DeviceArray
     (m, h), v = x.shape, len(w)
-    packed, y, best = DeviceArray((-(-v // 64) * 64, h), np.float32), DeviceArray((m, v), np.float32), DeviceArray((m,), np.uint64)
-    index = DeviceArray((m,), np.int64)
+    packed, y = DeviceArray((-(-v // 64) * 64, h), np.float32), DeviceArray((m, v), np.float32)
+    best, index = DeviceArray((m,), np.uint64), DeviceArray((m,), np.int64)
     hip.call("nc_pack_rows64", [packed, DeviceArray.from_host(w)], [v, h])
     hip.call("nc_argmax_clear", [best], [m])
     hip.call("nc_lm_head", [y, best, DeviceArray.from_host(x), packed], [m, v, h, 0, 0])

@@ -16,7 +16,8 @@ def run(tmp_path):
     """Compile and run a program over the rules; its output."""
     def go(body: str) -> str:
         source, binary = tmp_path / "rules.cpp", tmp_path / "rules"
-        source.write_text('#include <initializer_list>\n#include <stdio.h>\n#include "nc_rules.h"\nint main() {\n' + body + "\nreturn 0;\n}\n")
+        source.write_text('#include <initializer_list>\n#include <stdio.h>\n#include "nc_rules.h"\n'
+                          "int main() {\n" + body + "\nreturn 0;\n}\n")
         cxx = shutil.which("g++") or "c++"
         subprocess.run([cxx, "-O1", "-std=c++17", f"-I{CSRC}", "-o", str(binary), str(source)],
                        check=True)
@@ -123,10 +124,10 @@ def test_pair_tiles_where_they_are_quicker(run):
 
 def test_prompt_attention_where_the_matrix_cores_are_quicker(run):
     """Rows a workgroup of a prompt's attention: 4 (the vector ALU) where that measured quicker, else 0."""
-    vector = [(2, 8, 8, 2), (64, 8, 8, 64), (64, 8, 8, 464), (128, 4, 4, 528), (64, 16, 8, 164), (128, 12, 4, 128),
-              (64, 8, 2, 464), (128, 3, 3, 528), (8, 8, 8, 4008), (2, 66, 1, 2), (5000, 130, 2, 9000)]
-    matrix = [(64, 8, 8, 1264), (64, 4, 4, 1264), (128, 16, 8, 228), (256, 12, 4, 256), (128, 8, 2, 528), (512, 3, 3, 512),
-              (2, 14, 2, 2), (64, 24, 4, 64), (3, 64, 1, 133), (2048, 8, 8, 2048)]
+    vector = [(2, 8, 8, 2), (64, 8, 8, 64), (64, 8, 8, 464), (128, 4, 4, 528), (64, 16, 8, 164),
+              (128, 12, 4, 128), (64, 8, 2, 464), (128, 3, 3, 528), (8, 8, 8, 4008), (2, 66, 1, 2), (5000, 130, 2, 9000)]
+    matrix = [(64, 8, 8, 1264), (64, 4, 4, 1264), (128, 16, 8, 228), (256, 12, 4, 256), (128, 8, 2, 528),
+              (512, 3, 3, 512), (2, 14, 2, 2), (64, 24, 4, 64), (3, 64, 1, 133), (2048, 8, 8, 2048)]
     said = run("".join(f'printf("%d ", nc::prefill_rows({m}, {h}, {kv}, {keys}));'
                        for m, h, kv, keys in vector + matrix)).split()
     assert [s for s, r in zip(vector + matrix, said) if int(r) != (4 if s in vector else 0)] == []
